@@ -646,6 +646,14 @@ static ModalGrid modal_grid(const skt_operator* op, int k, int kc_block) {
   g.lz = nnz;
   const int64_t per = (int64_t)g.tiles_x * g.tiles_y * cblocks;
   while (g.lz > 6 && per * ((nnz + g.lz - 1) / g.lz) < 1024) g.lz = (g.lz + 1) / 2;
+  // Small grids: a launch lasts as long as one workgroup's walk through its
+  // chunk (2 to 3 us a layer), so shorter chunks down to single planes are
+  // taken until there are two workgroups per CU; the layers computed twice run
+  // on CUs that would be idle.  The 40x20x20 apply with 8 float32 columns went
+  // from 19 to 8 us, an OC iteration there from 5.57 to 4.67 ms; a target of
+  // 256 workgroups gave 4.86 ms, 1024 made 66x36x28 (3 float64 columns)
+  // slower, 8.5 to 9.2 ms.
+  while (g.lz > 1 && per * ((nnz + g.lz - 1) / g.lz) < 512) --g.lz;
   g.nzc = (int)((nnz + g.lz - 1) / g.lz);
   g.nblocks = per * g.nzc;
   return g;
