@@ -26,32 +26,103 @@ static int axis_factor(int64_t n) {
   return 1;
 }
 
-bool mg_plan(const skt_operator* op, const MGConfig& cfg, std::vector<MGLevel>* out) {
-  out->clear();
-  if (op->mesh != SKT_MESH_HEX8 && !(op->mesh == SKT_MESH_TET4 && op->tet_grid)) return false;
-  const int NC = op->ncomp;
+// Coarsening factors of a level by factors 2, 3 or 5 that divide its axes; an
+// axis is not collapsed to a single element while a longer axis (more than 5
+// elements) still coarsens: e.g. 15x5x5 -> 5x5x5, not 5x1x1.
+static bool divide_axes(const MGLevel& f, int (&fac)[3]) {
+  const int64_t n3[3] = {f.nx, f.ny, f.nz};
+  bool longer = false;
+  for (int a = 0; a < 3; ++a) {
+    fac[a] = axis_factor(n3[a]);
+    longer = longer || (n3[a] > 5 && fac[a] > 1);
+  }
+  if (longer)
+    for (int a = 0; a < 3; ++a)
+      if (fac[a] > 1 && n3[a] / fac[a] == 1) fac[a] = 1;
+  return fac[0] > 1 || fac[1] > 1 || fac[2] > 1;
+}
+
+// Factor 2 on every axis, whatever its length: the last coarse element of an
+// odd axis holds one fine element.  The same rule against collapsing.
+static bool halve_axes(const MGLevel& f, int (&fac)[3]) {
+  const int64_t n3[3] = {f.nx, f.ny, f.nz};
+  const bool longer = std::max(f.nx, std::max(f.ny, f.nz)) > 5;
+  for (int a = 0; a < 3; ++a) fac[a] = n3[a] > (longer ? 2 : 1) ? 2 : 1;
+  return fac[0] > 1 || fac[1] > 1 || fac[2] > 1;
+}
+
+static MGLevel coarser(const MGLevel& f, const int (&fac)[3], int NC) {
+  MGLevel c;
+  c.nx = (f.nx + fac[0] - 1) / fac[0];
+  c.ny = (f.ny + fac[1] - 1) / fac[1];
+  c.nz = (f.nz + fac[2] - 1) / fac[2];
+  for (int a = 0; a < 3; ++a) c.f[a] = fac[a];
+  c.nn = (c.nx + 1) * (c.ny + 1) * (c.nz + 1);
+  c.ndof = c.nn * NC;
+  return c;
+}
+
+static bool has_cell_grid(const skt_operator* op) {
+  return op->mesh == SKT_MESH_HEX8 || (op->mesh == SKT_MESH_TET4 && op->tet_grid);
+}
+
+static MGLevel fine_level(const skt_operator* op) {
   MGLevel l0;
   l0.nx = op->nx; l0.ny = op->ny; l0.nz = op->nz;
   l0.nn = (l0.nx + 1) * (l0.ny + 1) * (l0.nz + 1);
-  l0.ndof = l0.nn * NC;
-  out->push_back(l0);
+  l0.ndof = l0.nn * op->ncomp;
+  return l0;
+}
+
+bool mg_divides(const skt_operator* op, const MGConfig& cfg) {
+  if (!has_cell_grid(op)) return false;
+  MGLevel l = fine_level(op);
+  int n = 1;
+  for (; l.ndof > cfg.max_coarse; ++n) {
+    int fac[3];
+    if (!divide_axes(l, fac)) return false;
+    l = coarser(l, fac, op->ncomp);
+  }
+  return n >= 2;
+}
+
+bool mg_plan(const skt_operator* op, const MGConfig& cfg, std::vector<MGLevel>* out) {
+  out->clear();
+  if (!has_cell_grid(op)) return false;
+  out->push_back(fine_level(op));
+  // Conduction and mass operators take 8 to 16 iterations whatever the factors:
+  // they keep the fewest levels where factors 2, 3 and 5 divide the grid.
+  const bool few = op->ncomp == 1 && mg_divides(op, cfg);
   while (out->back().ndof > cfg.max_coarse) {
     const MGLevel& f = out->back();
-    int fac[3] = {axis_factor(f.nx), axis_factor(f.ny), axis_factor(f.nz)};
-    // an axis is not collapsed to a single element while a longer axis
-    // (more than 5 elements) still coarsens: e.g. 15x5x5 -> 5x5x5, not 5x1x1
-    const int64_t n3[3] = {f.nx, f.ny, f.nz};
-    bool longer = false;
-    for (int a = 0; a < 3; ++a) longer = longer || (n3[a] > 5 && fac[a] > 1);
-    if (longer)
-      for (int a = 0; a < 3; ++a)
-        if (fac[a] > 1 && n3[a] / fac[a] == 1) fac[a] = 1;
-    if (fac[0] == 1 && fac[1] == 1 && fac[2] == 1) return false;
-    MGLevel c;
-    c.nx = f.nx / fac[0]; c.ny = f.ny / fac[1]; c.nz = f.nz / fac[2];
-    c.f[0] = fac[0]; c.f[1] = fac[1]; c.f[2] = fac[2];
-    c.nn = (c.nx + 1) * (c.ny + 1) * (c.nz + 1);
-    c.ndof = c.nn * NC;
+    int fac[3];
+    // Levels above kDivideNodes nodes are halved on every axis.  Factors 3
+    // and 5 leave the smoother error it cannot reach and stretch the coarse
+    // elements where the axes take different factors; on smaller levels a
+    // level less is worth more than that.
+    const bool ok = few || f.nn <= kDivideNodes ? divide_axes(f, fac) || halve_axes(f, fac)
+                                                : halve_axes(f, fac);
+    if (!ok) return false;
+    MGLevel c = coarser(f, fac, op->ncomp);
+    // A coarsest level that fits with factor 3 on some axes, where halving
+    // them all does not: the largest such level.  One more halved level would
+    // leave a much smaller coarsest one, and the exact solve is what catches
+    // the error of stiff members in voids: 120x60x60, 8 loads, mixed, with
+    // 10x8x5 elements in place of 15x8x8 and 8x4x4 takes 24 PCG iterations
+    // per solve instead of 29 (18.6 against 21.2 ms per OC iteration).
+    if (c.ndof > cfg.max_coarse && f.nn > kDivideNodes && !few) {
+      const int64_t n3[3] = {f.nx, f.ny, f.nz};
+      int64_t best = 0;
+      for (int m = 1; m < 8; ++m) {
+        int g[3];
+        for (int a = 0; a < 3; ++a) g[a] = ((m >> a) & 1) && fac[a] == 2 && n3[a] >= 5 ? 3 : fac[a];
+        const MGLevel t = coarser(f, g, op->ncomp);
+        if (t.ndof <= cfg.max_coarse && t.ndof > best) {
+          best = t.ndof;
+          c = t;
+        }
+      }
+    }
     out->push_back(c);
   }
   return out->size() >= 2;
@@ -70,6 +141,13 @@ __device__ __forceinline__ double tri_weight(int q, int Q, int a, int b, int c, 
   const double wy = (Q & 2) ? sy : 1.0 - sy;
   const double wz = (Q & 4) ? sz : 1.0 - sz;
   return wx * wy * wz;
+}
+
+// Fine elements of coarse element C along an axis of nf fine elements: f, or
+// what is left at the end of the axis.
+__host__ __device__ inline int children(int64_t nf, int64_t C, int f) {
+  const int64_t left = nf - C * f;
+  return left < f ? (int)left : f;
 }
 
 // acc += P_j^T sK P_j for child (a, b, c) of a coarse element divided by
@@ -118,8 +196,8 @@ __device__ __forceinline__ void galerkin_child(const double* sK, double* sT, dou
 // flag is 0 are left to k_galerkin_interior.
 template <int NC>
 __global__ void __launch_bounds__(64)
-k_galerkin(int64_t ncx, int64_t ncy, int64_t ncz, int fx, int fy, int fz,
-           const double* __restrict__ Kf, const double* __restrict__ K0b,
+k_galerkin(int64_t ncx, int64_t ncy, int64_t ncz, int64_t nfx, int64_t nfy, int64_t nfz, int fx,
+           int fy, int fz, const double* __restrict__ Kf, const double* __restrict__ K0b,
            const double* __restrict__ E, const uint8_t* __restrict__ fixed,
            const uint8_t* __restrict__ only, double* __restrict__ Kc) {
   constexpr int ND = 8 * NC;
@@ -131,15 +209,15 @@ k_galerkin(int64_t ncx, int64_t ncy, int64_t ncz, int fx, int fy, int fz,
   const int64_t ce = blockIdx.x;
   if (only && !only[ce]) return;
   const int64_t CX = ce % ncx, CY = (ce / ncx) % ncy, CZ = ce / (ncx * ncy);
-  const int64_t nfx = ncx * fx, nfy = ncy * fy;
   const int64_t nfnx = nfx + 1, nfny = nfy + 1;
   const int tid = threadIdx.x;
+  const int cx = children(nfx, CX, fx), cy = children(nfy, CY, fy), cz = children(nfz, CZ, fz);
   double acc[PER];
 #pragma unroll
   for (int i = 0; i < PER; ++i) acc[i] = 0.0;
-  for (int c = 0; c < fz; ++c)
-    for (int b = 0; b < fy; ++b)
-      for (int a = 0; a < fx; ++a) {
+  for (int c = 0; c < cz; ++c)
+    for (int b = 0; b < cy; ++b)
+      for (int a = 0; a < cx; ++a) {
         const int64_t ex = CX * fx + a, ey = CY * fy + b, ez = CZ * fz + c;
         const int64_t fe = ex + nfx * (ey + nfy * ez);
         // child matrix
@@ -161,7 +239,7 @@ k_galerkin(int64_t ncx, int64_t ncy, int64_t ncz, int fx, int fy, int fz,
             sK[i] = v;
           }
         }
-        galerkin_child<NC>(sK, sT, sP, a, b, c, fx, fy, fz, acc);
+        galerkin_child<NC>(sK, sT, sP, a, b, c, cx, cy, cz, acc);
       }
 #pragma unroll
   for (int k = 0; k < PER; ++k) {
@@ -179,7 +257,8 @@ k_galerkin(int64_t ncx, int64_t ncy, int64_t ncz, int fx, int fy, int fz,
 // gradients, Z removing Dirichlet DOFs) and projected as the hex children.
 template <int NC>
 __global__ void __launch_bounds__(64)
-k_galerkin_tet(int64_t ncx, int64_t ncy, int64_t ncz, int fx, int fy, int fz,
+k_galerkin_tet(int64_t ncx, int64_t ncy, int64_t ncz, int64_t nfx, int64_t nfy, int64_t nfz,
+               int fx, int fy, int fz,
                const int32_t* __restrict__ conn, const double* __restrict__ g,
                const double* __restrict__ vol, double lam0, double mu0, int64_t n_el,
                const double* __restrict__ E, const uint8_t* __restrict__ fixed,
@@ -197,15 +276,15 @@ k_galerkin_tet(int64_t ncx, int64_t ncy, int64_t ncz, int fx, int fy, int fz,
   __shared__ uint8_t sfix[ND];    // the cell corners' Dirichlet flags
   const int64_t ce = blockIdx.x;
   const int64_t CX = ce % ncx, CY = (ce / ncx) % ncy, CZ = ce / (ncx * ncy);
-  const int64_t nfx = ncx * fx, nfy = ncy * fy;
   const int64_t nfnx = nfx + 1, nfny = nfy + 1;
   const int tid = threadIdx.x;
+  const int cx = children(nfx, CX, fx), cy = children(nfy, CY, fy), cz = children(nfz, CZ, fz);
   double acc[PER];
 #pragma unroll
   for (int i = 0; i < PER; ++i) acc[i] = 0.0;
-  for (int c = 0; c < fz; ++c)
-    for (int b = 0; b < fy; ++b)
-      for (int a = 0; a < fx; ++a) {
+  for (int c = 0; c < cz; ++c)
+    for (int b = 0; b < cy; ++b)
+      for (int a = 0; a < cx; ++a) {
         const int64_t ex = CX * fx + a, ey = CY * fy + b, ez = CZ * fz + c;
         const int64_t cell = ex + nfx * (ey + nfy * ez);
         // (the previous child's projection ended with a barrier)
@@ -251,7 +330,7 @@ k_galerkin_tet(int64_t ncx, int64_t ncy, int64_t ncz, int fx, int fy, int fz,
           }
           __syncthreads();
         }
-        galerkin_child<NC>(sK, sT, sP, a, b, c, fx, fy, fz, acc);
+        galerkin_child<NC>(sK, sT, sP, a, b, c, cx, cy, cz, acc);
       }
 #pragma unroll
   for (int k = 0; k < PER; ++k) {
@@ -289,19 +368,22 @@ k_galerkin_children(int fx, int fy, int fz, const double* __restrict__ K0b,
 }
 
 // 1 for the coarse elements of the first coarse level whose fine nodes hold
-// a Dirichlet DOF (their children need the masked product), else 0.
+// a Dirichlet DOF (their children need the masked product; fixed may be null)
+// or that hold fewer fine elements than the others, else 0.
 template <int NC>
-__global__ void k_galerkin_flags(int64_t ncx, int64_t ncy, int64_t ncz, int fx, int fy, int fz,
+__global__ void k_galerkin_flags(int64_t ncx, int64_t ncy, int64_t ncz, int64_t nfx, int64_t nfy,
+                                 int64_t nfz, int fx, int fy, int fz,
                                  const uint8_t* __restrict__ fixed, uint8_t* __restrict__ flag) {
   const int64_t nce = ncx * ncy * ncz;
-  const int64_t nfnx = ncx * fx + 1, nfny = ncy * fy + 1;
+  const int64_t nfnx = nfx + 1, nfny = nfy + 1;
   for (int64_t ce = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; ce < nce;
        ce += (int64_t)gridDim.x * blockDim.x) {
     const int64_t CX = ce % ncx, CY = (ce / ncx) % ncy, CZ = ce / (ncx * ncy);
-    uint8_t any = 0;
-    for (int k = 0; k <= fz; ++k)
-      for (int j = 0; j <= fy; ++j)
-        for (int i = 0; i <= fx; ++i) {
+    const int cx = children(nfx, CX, fx), cy = children(nfy, CY, fy), cz = children(nfz, CZ, fz);
+    uint8_t any = cx < fx || cy < fy || cz < fz;
+    for (int k = 0; k <= cz && fixed; ++k)
+      for (int j = 0; j <= cy; ++j)
+        for (int i = 0; i <= cx; ++i) {
           const int64_t n = (CX * fx + i) + nfnx * ((CY * fy + j) + nfny * (CZ * fz + k));
 #pragma unroll
           for (int d = 0; d < NC; ++d) any |= fixed[n * NC + d];
@@ -310,20 +392,20 @@ __global__ void k_galerkin_flags(int64_t ncx, int64_t ncy, int64_t ncz, int fx, 
   }
 }
 
-// Kc = sum_j E_j M_j for the coarse elements without Dirichlet DOFs (flag
-// null: all of them).  A workgroup of NN threads (one per entry) walks over
+// Kc = sum_j E_j M_j for the coarse elements without Dirichlet DOFs and with
+// all their fine elements (flag null: all of them).  A workgroup of NN threads (one per entry) walks over
 // coarse elements, with the element's child moduli staged in LDS; the
 // children are summed in the order k_galerkin takes them.
 constexpr int kMaxChildren = 125;  // factor 5 on every axis
 template <int NC>
 __global__ void __launch_bounds__(64 * NC * NC)
-k_galerkin_interior(int64_t ncx, int64_t ncy, int64_t ncz, int fx, int fy, int fz,
+k_galerkin_interior(int64_t ncx, int64_t ncy, int64_t ncz, int64_t nfx, int64_t nfy, int fx,
+                    int fy, int fz,
                     const double* __restrict__ M, const double* __restrict__ E,
                     const uint8_t* __restrict__ flag, double* __restrict__ Kc) {
   constexpr int NN = 64 * NC * NC;
   __shared__ double sE[kMaxChildren];
   const int64_t nce = ncx * ncy * ncz;
-  const int64_t nfx = ncx * fx, nfy = ncy * fy;
   const int nch = fx * fy * fz;
   const int tid = threadIdx.x;
   for (int64_t ce = blockIdx.x; ce < nce; ce += gridDim.x) {
@@ -1060,16 +1142,37 @@ static RowGrid row_grid(int64_t row_len, int64_t rows) {
 // Restriction b_c = P^T Z (b - w), separable in two passes.
 // Pass 1 (x, y): t[(I, J, k)] = sum_{dx,dy} w(dx) w(dy) r(f I + dx, f J + dy, k)
 // on every fine z plane k, r = b - w with Dirichlet DOFs removed.  Thread:
-// coarse I; row: (J, k, group).
+// coarse I; row: (J, k, group).  The coarse node at the end of an axis lies
+// on the axis' last fine node, wl fine elements from its neighbour.
+__device__ __forceinline__ int interval(int fn, int I, int f) {
+  // fine elements right of coarse node I, f past the last one
+  const int left = fn - I * f;
+  return left > 0 && left < f ? left : f;
+}
+
+struct Taps {
+  int x, wl, wr;  // fine position, fine elements to the left and right neighbour
+};
+
+__device__ __forceinline__ Taps coarse_taps(int I, int f, int fn) {
+  Taps t;
+  t.x = I * f < fn ? I * f : fn;
+  t.wl = I > 0 ? t.x - (I - 1) * f : 1;
+  const int right = fn - t.x;
+  t.wr = right < f ? (right > 0 ? right : 1) : f;
+  return t;
+}
+
 template <typename T, int NC, int KC>
 __global__ void k_restrict_xy(int fnx, int fny, int fnz, int fx, int fy, int groups,
                               const T* __restrict__ b, const T* __restrict__ w,
                               const uint8_t* __restrict__ fixed, T* __restrict__ tbuf) {
   const int fnnx = fnx + 1, fnny = fny + 1, fnnz = fnz + 1;
-  const int cnnx = fnx / fx + 1, cnny = fny / fy + 1;
+  const int cnnx = (fnx + fx - 1) / fx + 1, cnny = (fny + fy - 1) / fy + 1;
   const int64_t tn = (int64_t)cnnx * cnny * fnnz, fnn = (int64_t)fnnx * fnny * fnnz;
   const int I = blockIdx.x * blockDim.x + threadIdx.x;
   if (I >= cnnx) return;
+  const Taps tx = coarse_taps(I, fx, fnx);
   const int nrows = cnny * fnnz * groups;
   for (int row = blockIdx.y; row < nrows; row += gridDim.y) {
     const int J = row % cnny, kg = row / cnny, k = kg % fnnz, g = kg / fnnz;
@@ -1080,14 +1183,13 @@ __global__ void k_restrict_xy(int fnx, int fny, int fnz, int fx, int fy, int gro
     for (int d = 0; d < NC; ++d)
 #pragma unroll
       for (int c = 0; c < KC; ++c) acc[d][c] = T(0);
-    for (int dy = -(fy - 1); dy <= fy - 1; ++dy) {
-      const int j = J * fy + dy;
-      if (j < 0 || j >= fnny) continue;
-      const T wy = T(1) - (T)(dy < 0 ? -dy : dy) / (T)fy;
-      for (int dx = -(fx - 1); dx <= fx - 1; ++dx) {
-        const int i = I * fx + dx;
-        if (i < 0 || i >= fnnx) continue;
-        const T wgt = (T(1) - (T)(dx < 0 ? -dx : dx) / (T)fx) * wy;
+    const Taps ty = coarse_taps(J, fy, fny);
+    for (int dy = 1 - ty.wl; dy <= ty.wr - 1; ++dy) {
+      const int j = ty.x + dy;
+      const T wy = T(1) - (dy < 0 ? (T)-dy / (T)ty.wl : (T)dy / (T)ty.wr);
+      for (int dx = 1 - tx.wl; dx <= tx.wr - 1; ++dx) {
+        const int i = tx.x + dx;
+        const T wgt = (T(1) - (dx < 0 ? (T)-dx / (T)tx.wl : (T)dx / (T)tx.wr)) * wy;
         const int64_t fn = i + fnnx * (j + (int64_t)fnny * k);
         T bv[NC * KC], wv[NC * KC];
         load_node<T, NC * KC, KC>(bg + fn * NC * KC, bv);
@@ -1115,7 +1217,7 @@ __global__ void k_restrict_xy(int fnx, int fny, int fnz, int fx, int fy, int gro
 template <typename T, int NC, int KC>
 __global__ void k_restrict_z(int cnnx, int cnny, int fnz, int fz, int groups,
                              const T* __restrict__ tbuf, T* __restrict__ bc) {
-  const int fnnz = fnz + 1, cnnz = fnz / fz + 1;
+  const int fnnz = fnz + 1, cnnz = (fnz + fz - 1) / fz + 1;
   const int64_t plane = (int64_t)cnnx * cnny;
   const int64_t tn = plane * fnnz, cnn = plane * cnnz;
   const int64_t IJ = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
@@ -1129,10 +1231,10 @@ __global__ void k_restrict_z(int cnnx, int cnny, int fnz, int fz, int groups,
     for (int d = 0; d < NC; ++d)
 #pragma unroll
       for (int c = 0; c < KC; ++c) acc[d][c] = T(0);
-    for (int dz = -(fz - 1); dz <= fz - 1; ++dz) {
-      const int k = K * fz + dz;
-      if (k < 0 || k >= fnnz) continue;
-      const T wz = T(1) - (T)(dz < 0 ? -dz : dz) / (T)fz;
+    const Taps tz = coarse_taps(K, fz, fnz);
+    for (int dz = 1 - tz.wl; dz <= tz.wr - 1; ++dz) {
+      const int k = tz.x + dz;
+      const T wz = T(1) - (dz < 0 ? (T)-dz / (T)tz.wl : (T)dz / (T)tz.wr);
       const int64_t tnode = IJ + plane * k;
 #pragma unroll
       for (int d = 0; d < NC; ++d)
@@ -1161,7 +1263,9 @@ __global__ void k_restrict_z(int cnnx, int cnny, int fnz, int fz, int groups,
 // mask is applied: b must be zero at Dirichlet DOFs (the fine residual is) or
 // there are none (coarse levels).  With x0 the kernel also writes the coarse
 // level's first smoothing iterate from zero, x0 = c2 dinv_c b_c (k_cheb_first
-// with c2 = cf[1]).
+// with c2 = cf[1]).  On an axis of odd length the last coarse node lies on the
+// last fine node, the dx = -1 neighbour of where it would be: it takes that
+// node with weight 1, and the coarse node before it has no dx = +1 neighbour.
 constexpr int kR2I = 32, kR2J = 8;
 
 template <typename T, int NC, int KC, bool HASW>
@@ -1177,7 +1281,7 @@ k_restrict222(int fnx, int fny, int fnz, int tiles_x, int tiles_y, int zchunks, 
   constexpr int kQ = (kH + 3) / 4;                       // rows per wavefront
   __shared__ T sv[NV * kH * kW];                         // [value][row][node]
   const int fnnx = fnx + 1, fnny = fny + 1, fnnz = fnz + 1;
-  const int cnnx = fnx / 2 + 1, cnny = fny / 2 + 1, cnnz = fnz / 2 + 1;
+  const int cnnx = (fnx + 1) / 2 + 1, cnny = (fny + 1) / 2 + 1, cnnz = (fnz + 1) / 2 + 1;
   const int64_t fnn = (int64_t)fnnx * fnny * fnnz, cnn = (int64_t)cnnx * cnny * cnnz;
   int blk = blockIdx.x;
   const int tx = blk % tiles_x;
@@ -1239,6 +1343,8 @@ k_restrict222(int fnx, int fny, int fnz, int tiles_x, int tiles_y, int zchunks, 
   const int Il = tid % kR2I, Jl = tid / kR2I;
   const int I = tx * kR2I + Il, J = ty * kR2J + Jl;
   const bool own = I < cnnx && J < cnny;
+  const T xl = 2 * I > fnx ? T(1) : T(0.5), xr = 2 * I + 1 == fnx ? T(0) : T(0.5);
+  const T yl = 2 * J > fny ? T(1) : T(0.5), yr = 2 * J + 1 == fny ? T(0) : T(0.5);
   T acc[NV];
 #pragma unroll
   for (int v = 0; v < NV; ++v) acc[v] = T(0);
@@ -1269,10 +1375,10 @@ k_restrict222(int fnx, int fny, int fnz, int tiles_x, int tiles_y, int zchunks, 
     if (have) {
 #pragma unroll
       for (int dy = -1; dy <= 1; ++dy) {
-        const T wy = T(1) - (T)(dy < 0 ? -dy : dy) / T(2);
+        const T wy = dy < 0 ? yl : dy > 0 ? yr : T(1);
 #pragma unroll
         for (int dx = -1; dx <= 1; ++dx) {
-          const T wgt = (T(1) - (T)(dx < 0 ? -dx : dx) / T(2)) * wy;
+          const T wgt = (dx < 0 ? xl : dx > 0 ? xr : T(1)) * wy;
           const int node = (2 * Jl + 1 + dy) * kW + 2 * Il + 1 + dx;
 #pragma unroll
           for (int v = 0; v < NV; ++v) t[v] += wgt * sv[v * kH * kW + node];
@@ -1284,8 +1390,9 @@ k_restrict222(int fnx, int fny, int fnz, int tiles_x, int tiles_y, int zchunks, 
     // this order, as k_restrict_z sums them)
     if (gz & 1) {
       const int K = (gz - 1) >> 1;  // dz = +1 for K, -1 for K + 1
+      const bool end = gz == fnz;   // the last coarse plane lies on this one
       if (K >= K0) {
-        if (have) {
+        if (have && !end) {
 #pragma unroll
           for (int v = 0; v < NV; ++v) acc[v] += T(0.5) * t[v];
         }
@@ -1294,8 +1401,10 @@ k_restrict222(int fnx, int fny, int fnz, int tiles_x, int tiles_y, int zchunks, 
 #pragma unroll
       for (int v = 0; v < NV; ++v) acc[v] = T(0);
       if (have && K + 1 < K1) {
+        const T wz = end ? T(1) : T(0.5);
 #pragma unroll
-        for (int v = 0; v < NV; ++v) acc[v] += T(0.5) * t[v];
+        for (int v = 0; v < NV; ++v) acc[v] += wz * t[v];
+        if (end) write(K + 1);
       }
     } else {
       const int K = gz >> 1;
@@ -1318,17 +1427,19 @@ __global__ void k_prolong_add(int fnx, int fny, int fnz, int fx, int fy, int fz,
                               const T* __restrict__ xc, const uint8_t* __restrict__ fixed,
                               T* __restrict__ xf) {
   const int fnnx = fnx + 1, fnny = fny + 1, fnnz = fnz + 1;
-  const int cnnx = fnx / fx + 1, cnny = fny / fy + 1, cnnz = fnz / fz + 1;
+  const int cnnx = (fnx + fx - 1) / fx + 1, cnny = (fny + fy - 1) / fy + 1,
+            cnnz = (fnz + fz - 1) / fz + 1;
   const int64_t cnn = (int64_t)cnnx * cnny * cnnz, fnn = (int64_t)fnnx * fnny * fnnz;
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= fnnx) return;
+  // the coarse element at the end of an axis may hold fewer fine elements
   const int I = i / fx, ax = i - I * fx;
-  const T sx = (T)ax / (T)fx;
+  const T sx = (T)ax / (T)interval(fnx, I, fx);
   const int nrows = fnny * fnnz * groups;
   for (int row = blockIdx.y; row < nrows; row += gridDim.y) {
     const int j = row % fnny, kg = row / fnny, k = kg % fnnz, g = kg / fnnz;
     const int J = j / fy, ay = j - J * fy, K = k / fz, az = k - K * fz;
-    const T sy = (T)ay / (T)fy, sz = (T)az / (T)fz;
+    const T sy = (T)ay / (T)interval(fny, J, fy), sz = (T)az / (T)interval(fnz, K, fz);
     const int64_t fnode = i + fnnx * (j + (int64_t)fnny * k);
     const T* xg = xc + g * cnn * NC * KC;
     T* xfn = xf + (g * fnn + fnode) * NC * KC;
@@ -1614,13 +1725,13 @@ __global__ void k_pow_scale(int64_t n, const double* __restrict__ inv, const T* 
 }
 
 // Chebyshev (c1, c2) per step for the interval [beta/ratio, beta],
-// beta = 1.1 * lambda estimate
-__global__ void k_cheb_coef(int nlev, int degree, double ratio, const double* __restrict__ lam,
-                            double* __restrict__ coef) {
+// beta = 1.1 * lambda estimate; the last level takes ratio_low
+__global__ void k_cheb_coef(int nlev, int degree, double ratio, double ratio_low,
+                            const double* __restrict__ lam, double* __restrict__ coef) {
   const int l = threadIdx.x;
   if (l >= nlev) return;
   const double bmax = 1.1 * lam[l];
-  const double amin = bmax / ratio;
+  const double amin = bmax / (l > 0 && l == nlev - 1 ? ratio_low : ratio);
   const double theta = 0.5 * (bmax + amin), delta = 0.5 * (bmax - amin);
   const double sigma = theta / delta;
   double* c = coef + (size_t)l * 2 * degree;
@@ -1636,6 +1747,9 @@ __global__ void k_cheb_coef(int nlev, int degree, double ratio, const double* __
 }
 
 // ------------------------------------------------------------ host side
+
+// Chebyshev steps whose coefficients are kept per level
+static int coef_steps(const MGData* mg) { return mg->degree + kLowSteps; }
 
 static size_t tsize(int dtype) { return dtype == SKT_F64 ? sizeof(double) : sizeof(float); }
 
@@ -1747,7 +1861,7 @@ int mg_alloc(MGData* mg, const skt_operator* op, const MGConfig& cfg, int dtype,
                 (op->ny + 1) * (op->nz + 1) * (int64_t)max_cols < INT32_MAX,
             "grid too large for the multigrid transfers' 32-bit row indices");
   mg_free(mg);
-  std::vector<MGLevel> lv;
+  std::vector<MGLevel>& lv = mg->lv;  // mg_free returns what a failed call allocated
   if (!mg_plan(op, cfg, &lv)) {
     set_error("grid cannot be coarsened for multigrid");
     return SKT_EINVAL;
@@ -1780,7 +1894,7 @@ int mg_alloc(MGData* mg, const skt_operator* op, const MGConfig& cfg, int dtype,
   SKT_HIP(hipMalloc(&mg->Ad2, sizeof(double) * 2 * kGJ * kGJ));
   SKT_HIP(hipMalloc(&mg->Ainv, ts * nc * nc));
   SKT_HIP(hipMalloc(&mg->lam, sizeof(double) * (L + 1) * 2));
-  SKT_HIP(hipMalloc(&mg->coef, sizeof(double) * (L + 1) * 2 * std::max(cfg.degree, 1)));
+  SKT_HIP(hipMalloc(&mg->coef, sizeof(double) * (L + 1) * 2 * (std::max(cfg.degree, 1) + kLowSteps)));
   SKT_HIP(hipMalloc(&mg->part, sizeof(double) * 1024));
   SKT_HIP(hipMalloc(&mg->pv, ts * 2 * lv[0].ndof));
   int64_t npw = 0;
@@ -1799,12 +1913,12 @@ int mg_alloc(MGData* mg, const skt_operator* op, const MGConfig& cfg, int dtype,
     }
   SKT_HIP(hipMalloc(&mg->K0b, sizeof(double) * K0b.size()));
   SKT_HIP(hipMemcpy(mg->K0b, K0b.data(), sizeof(double) * K0b.size(), hipMemcpyHostToDevice));
-  mg->lv = lv;
   mg->dtype = dtype;
   ++mg->gen;
   mg->max_cols = max_cols;
   mg->degree = std::max(cfg.degree, 1);
-  mg->ratio = cfg.ratio;
+  mg->low_steps = NC == 3 ? kLowSteps : 0;
+  mg->ratio = NC == 3 ? cfg.ratio : cfg.ratio_scalar;
   if (const char* rv = std::getenv("SKT_MG_RATIO")) {  // smoothing interval [lambda/r, lambda]
     const double r = std::atof(rv);
     if (r > 1.0 && r < 1000.0) mg->ratio = r;
@@ -1993,17 +2107,17 @@ static int setup_t(MGData* mg, const skt_operator* op, const double* E64, const 
   // Galerkin hierarchy.  The first coarse level takes E_j M_j for its
   // interior elements (M_j and the boundary flags depend on the operator
   // only, so they are built once) and the masked product for the rest.
+  const uint8_t* fx0 = op->n_fixed > 0 ? op->fixed : nullptr;
   if (op->mesh == SKT_MESH_TET4) {
     const MGLevel& c = mg->lv[1];
     const int64_t nce = c.nx * c.ny * c.nz;
-    const uint8_t* fx0 = op->n_fixed > 0 ? op->fixed : nullptr;
     if (NC == 3)
       hipLaunchKernelGGL((k_galerkin_tet<3>), dim3((unsigned)nce), dim3(64), 0, g, c.nx, c.ny,
-                         c.nz, c.f[0], c.f[1], c.f[2], op->conn, op->g64, op->vol64, op->lam0,
+                         c.nz, op->nx, op->ny, op->nz, c.f[0], c.f[1], c.f[2], op->conn, op->g64, op->vol64, op->lam0,
                          op->mu0, op->n_el, E64, fx0, c.Kel);
     else
       hipLaunchKernelGGL((k_galerkin_tet<1>), dim3((unsigned)nce), dim3(64), 0, g, c.nx, c.ny,
-                         c.nz, c.f[0], c.f[1], c.f[2], op->conn, op->g64, op->vol64, op->lam0,
+                         c.nz, op->nx, op->ny, op->nz, c.f[0], c.f[1], c.f[2], op->conn, op->g64, op->vol64, op->lam0,
                          op->mu0, op->n_el, E64, fx0, c.Kel);
     SKT_LAUNCH_CHECK();
   } else {
@@ -2018,14 +2132,18 @@ static int setup_t(MGData* mg, const skt_operator* op, const double* E64, const 
       else
         hipLaunchKernelGGL((k_galerkin_children<1>), dim3(nch), dim3(64), 0, g, c.f[0], c.f[1],
                            c.f[2], dK0, mg->Mch);
-      if (op->n_fixed > 0) {
+      const bool ragged = c.nx * c.f[0] != op->nx || c.ny * c.f[1] != op->ny ||
+                          c.nz * c.f[2] != op->nz;
+      if (op->n_fixed > 0 || ragged) {
         SKT_HIP(hipMalloc(&mg->gflag, (size_t)nce));
         if (NC == 3)
           hipLaunchKernelGGL((k_galerkin_flags<3>), dim3(grid_for(nce)), dim3(kBlock), 0, g,
-                             c.nx, c.ny, c.nz, c.f[0], c.f[1], c.f[2], op->fixed, mg->gflag);
+                             c.nx, c.ny, c.nz, op->nx, op->ny, op->nz, c.f[0], c.f[1], c.f[2], fx0,
+                             mg->gflag);
         else
           hipLaunchKernelGGL((k_galerkin_flags<1>), dim3(grid_for(nce)), dim3(kBlock), 0, g,
-                             c.nx, c.ny, c.nz, c.f[0], c.f[1], c.f[2], op->fixed, mg->gflag);
+                             c.nx, c.ny, c.nz, op->nx, op->ny, op->nz, c.f[0], c.f[1], c.f[2], fx0,
+                             mg->gflag);
       }
       SKT_LAUNCH_CHECK();
     }
@@ -2033,34 +2151,34 @@ static int setup_t(MGData* mg, const skt_operator* op, const double* E64, const 
     const unsigned gi = (unsigned)std::min<int64_t>(nce, 8192);
     if (NC == 3)
       hipLaunchKernelGGL((k_galerkin_interior<3>), dim3(gi), dim3(64 * 9), 0, g, c.nx, c.ny, c.nz,
-                         c.f[0], c.f[1], c.f[2], mg->Mch, E64, mg->gflag, c.Kel);
+                         op->nx, op->ny, c.f[0], c.f[1], c.f[2], mg->Mch, E64, mg->gflag, c.Kel);
     else
       hipLaunchKernelGGL((k_galerkin_interior<1>), dim3(gi), dim3(64), 0, g, c.nx, c.ny, c.nz,
-                         c.f[0], c.f[1], c.f[2], mg->Mch, E64, mg->gflag, c.Kel);
+                         op->nx, op->ny, c.f[0], c.f[1], c.f[2], mg->Mch, E64, mg->gflag, c.Kel);
     if (mg->gflag) {
       if (NC == 3)
         hipLaunchKernelGGL((k_galerkin<3>), dim3((unsigned)nce), dim3(64), 0, g, c.nx, c.ny,
-                           c.nz, c.f[0], c.f[1], c.f[2], nullptr, dK0, E64, op->fixed,
-                           mg->gflag, c.Kel);
+                           c.nz, op->nx, op->ny, op->nz, c.f[0], c.f[1], c.f[2], nullptr, dK0,
+                           E64, fx0, mg->gflag, c.Kel);
       else
         hipLaunchKernelGGL((k_galerkin<1>), dim3((unsigned)nce), dim3(64), 0, g, c.nx, c.ny,
-                           c.nz, c.f[0], c.f[1], c.f[2], nullptr, dK0, E64, op->fixed,
-                           mg->gflag, c.Kel);
+                           c.nz, op->nx, op->ny, op->nz, c.f[0], c.f[1], c.f[2], nullptr, dK0,
+                           E64, fx0, mg->gflag, c.Kel);
     }
     SKT_LAUNCH_CHECK();
   }
   for (int l = 2; l <= L; ++l) {
     // the stencil levels' products are done: side2 may start
     if (l == L) SKT_HIP(hipEventRecord(mg->ev_gal, g));
-    const MGLevel& c = mg->lv[l];
+    const MGLevel &c = mg->lv[l], &f = mg->lv[l - 1];
     const int64_t nce = c.nx * c.ny * c.nz;
-    const double* Kf = mg->lv[l - 1].Kel;
+    const double* Kf = f.Kel;
     if (NC == 3)
       hipLaunchKernelGGL((k_galerkin<3>), dim3((unsigned)nce), dim3(64), 0, g, c.nx, c.ny, c.nz,
-                         c.f[0], c.f[1], c.f[2], Kf, dK0, E64, nullptr, nullptr, c.Kel);
+                         f.nx, f.ny, f.nz, c.f[0], c.f[1], c.f[2], Kf, dK0, E64, nullptr, nullptr, c.Kel);
     else
       hipLaunchKernelGGL((k_galerkin<1>), dim3((unsigned)nce), dim3(64), 0, g, c.nx, c.ny, c.nz,
-                         c.f[0], c.f[1], c.f[2], Kf, dK0, E64, nullptr, nullptr, c.Kel);
+                         f.nx, f.ny, f.nz, c.f[0], c.f[1], c.f[2], Kf, dK0, E64, nullptr, nullptr, c.Kel);
     SKT_LAUNCH_CHECK();
   }
   if (L < 2) SKT_HIP(hipEventRecord(mg->ev_gal, g));
@@ -2168,7 +2286,8 @@ static int setup_t(MGData* mg, const skt_operator* op, const double* E64, const 
     if (int stt = queue_coarsest()) return stt;
   }
   mg->warm = 1;
-  hipLaunchKernelGGL(k_cheb_coef, dim3(1), dim3(64), 0, s, L, mg->degree, mg->ratio, mg->lam,
+  hipLaunchKernelGGL(k_cheb_coef, dim3(1), dim3(64), 0, s, L, coef_steps(mg), mg->ratio,
+                     mg->low_steps ? std::max(mg->ratio, kLowRatio) : mg->ratio, mg->lam,
                      mg->coef);
   SKT_LAUNCH_CHECK();
   // every side-stream branch joins the main stream before the set-up
@@ -2260,6 +2379,11 @@ const float* modal_coef<float>(const skt_operator* op) { return op->modal_f; }
 // the difference of the two buffers, so no direction vector is kept.  The
 // number of fused steps, 2 * degree - 1, is odd: starting in lv[0].x the
 // cycle ends in z.
+// Smoothing steps of level l
+static int level_steps(const MGData* mg, int l) {
+  return mg->degree + (l > 0 && l + 2 == (int)mg->lv.size() ? mg->low_steps : 0);
+}
+
 template <typename T, int NC, int KC>
 static int vcycle_t(MGData* mg, const skt_operator* op, const void* E, const void* dinv0, int k,
                     const T* r, T* z, T* w0, hipStream_t s, double* dot, int max_slots,
@@ -2268,7 +2392,7 @@ static int vcycle_t(MGData* mg, const skt_operator* op, const void* E, const voi
   ost.stop = stop;
   const int L = (int)mg->lv.size() - 1;
   const int groups = k / KC;
-  const int deg = mg->degree;
+  const int deg = mg->degree, cs = coef_steps(mg);
   const uint8_t* fixed0 = op->n_fixed > 0 ? op->fixed : nullptr;
   const T* coef0 = modal_coef<T>(op);
   const T* E0 = (const T*)E;
@@ -2307,7 +2431,7 @@ static int vcycle_t(MGData* mg, const skt_operator* op, const void* E, const voi
     hipLaunchKernelGGL(k_rsub<T>, dim3(ge), dim3(kBlock), 0, s, total, v.ndof, KC, fixed0, r, w0);
     T* x01 = L > 1 ? (T*)mg->lv[1].x : nullptr;
     if (launch_restrict_fused<T, NC, KC>(v, mg->lv[1], groups, (const T*)w0, (const T*)nullptr,
-                                         (T*)mg->lv[1].b, mg->coef + (size_t)2 * deg, x01, s))
+                                         (T*)mg->lv[1].b, mg->coef + (size_t)2 * cs, x01, s))
       x0_done[1] = x01 != nullptr;
     else
       launch_restrict<T, NC, KC>(v, mg->lv[1], groups, (const T*)w0, (const T*)nullptr, fixed0,
@@ -2350,7 +2474,7 @@ static int vcycle_t(MGData* mg, const skt_operator* op, const void* E, const voi
     // coarsest
     T* x01 = L > 1 ? (T*)mg->lv[1].x : nullptr;
     if (launch_restrict_fused<T, NC, KC>(v, mg->lv[1], groups, (const T*)w0, (const T*)nullptr,
-                                         (T*)mg->lv[1].b, mg->coef + (size_t)2 * deg, x01, s))
+                                         (T*)mg->lv[1].b, mg->coef + (size_t)2 * cs, x01, s))
       x0_done[1] = x01 != nullptr;
     else
       launch_restrict<T, NC, KC>(v, mg->lv[1], groups, (const T*)w0, (const T*)nullptr, fixed0,
@@ -2367,13 +2491,13 @@ static int vcycle_t(MGData* mg, const skt_operator* op, const void* E, const voi
     T* B = (T*)v.d;
     T* w = (T*)v.w;
     const int64_t total = v.ndof * k;
-    const double* cf = mg->coef + (size_t)l * 2 * deg;
+    const double* cf = mg->coef + (size_t)l * 2 * cs;
     // step 0 from a zero iterate (formed by the fused restriction into this
     // level, or here), then fused steps (the iterate before step 0 is zero)
     if (!x0_done[l])
       hipLaunchKernelGGL(k_cheb_first<T>, dim3(grid_for(total)), dim3(kBlock), 0, s, total,
                          v.ndof, KC, cf, b, (const T*)v.dinv, A);
-    for (int st = 1; st < deg; ++st) {
+    for (int st = 1; st < level_steps(mg, l); ++st) {
       if ((stt = level_cheb<T>(mg, op, l, k, KC, A, B, cf + 2 * st, st == 1 ? 1 : 0, s, stop)))
         return stt;
       std::swap(A, B);
@@ -2382,7 +2506,7 @@ static int vcycle_t(MGData* mg, const skt_operator* op, const void* E, const voi
     if ((stt = level_apply<T>(mg, op, E, l, k, KC, A, w, s, ost))) return stt;
     T* x0n = l + 1 < L ? (T*)mg->lv[l + 1].x : nullptr;
     if (launch_restrict_fused<T, NC, KC>(v, mg->lv[l + 1], groups, b, w, (T*)mg->lv[l + 1].b,
-                                         mg->coef + (size_t)(l + 1) * 2 * deg, x0n, s))
+                                         mg->coef + (size_t)(l + 1) * 2 * cs, x0n, s))
       x0_done[l + 1] = x0n != nullptr;
     else
       launch_restrict<T, NC, KC>(v, mg->lv[l + 1], groups, b, w, nullptr, (T*)mg->lv[l + 1].b,
@@ -2401,9 +2525,9 @@ static int vcycle_t(MGData* mg, const skt_operator* op, const void* E, const voi
     MGLevel& v = mg->lv[l];
     T* A = it[l];
     T* B = (A == (T*)v.x) ? (T*)v.d : (T*)v.x;
-    const double* cf = mg->coef + (size_t)l * 2 * deg;
+    const double* cf = mg->coef + (size_t)l * 2 * cs;
     launch_prolong<T, NC, KC>(v, mg->lv[l + 1], groups, (const T*)it[l + 1], nullptr, A, s);
-    for (int st = 0; st < deg; ++st) {
+    for (int st = 0; st < level_steps(mg, l); ++st) {
       // step 0 has c1 = 0 and needs no previous iterate
       if ((stt = level_cheb<T>(mg, op, l, k, KC, A, B, cf + 2 * st, st == 0 ? 1 : 0, s, stop)))
         return stt;

@@ -1,8 +1,9 @@
 // Geometric multigrid preconditioner for structured hex8 operators (internal).
 //
 // Level 0 is the matrix-free fine operator.  Each coarser level groups
-// fx*fy*fz fine elements into one coarse element (factors 2, 3 or 5 per axis,
-// 1 where an axis cannot be divided) and carries the exact Galerkin operator
+// fx*fy*fz fine elements into one coarse element (factor 2 per axis, or 3 or 5
+// on small levels, 1 where an axis stays as it is; the last coarse element of
+// an axis takes what is left) and carries the exact Galerkin operator
 // P^T A P of trilinear interpolation, built element by element: the coarse
 // element matrix is sum_children P_c^T K_c P_c, with the fine Dirichlet rows
 // and columns removed first, so the hierarchy preconditions the operator on
@@ -41,6 +42,19 @@ struct MGLevel {
 // ones the small tiles.
 constexpr int64_t kTiledNodes = 20000;
 
+// Levels with at most this many nodes are coarsened by the factors 2, 3 or 5
+// that divide them (fewer levels), larger ones by 2.
+constexpr int64_t kDivideNodes = 1024;
+
+// In elasticity the last level above the coarsest takes kLowSteps more
+// smoothing steps than the others, on the interval [lambda/kLowRatio, lambda]: its applies cost
+// little beside the fine level's (120x60x60, 8 loads, mixed: 15.5 ms per OC
+// iteration at 20 PCG iterations, against 18.6 at 24 with two steps on
+// [lambda/10, lambda] everywhere; 6 steps gave 15.0 there, but more time on
+// small grids and, now and then, a cycle that is not positive definite).
+constexpr int kLowSteps = 2;
+constexpr double kLowRatio = 30.0;
+
 struct MGData {
   int dtype = -1;                     // SKT_F64 / SKT_F32 the buffers hold
   int max_cols = 0;
@@ -62,7 +76,8 @@ struct MGData {
                                       // normalised power-iteration vector in T
   int warm = 0;                       // pvw holds vectors from an earlier set-up
   int degree = 2;
-  double ratio = 10.0;
+  double ratio = 14.0;
+  int low_steps = 0;
   int power_iters = 20;               // steps from the hashed start vector
   int power_iters_warm = 5;           // steps from the previous set-up's vector
   uint64_t gen = 0;                   // bumped whenever the buffers are (re)allocated
@@ -101,13 +116,20 @@ enum { MG_T_CHEB0 = 0, MG_T_RESID = 1, MG_T_CHEB = 2, MG_T_CHEB_DOT = 3 };
 struct MGConfig {
   int degree = 2;          // Chebyshev steps per smoothing
   int max_coarse = 2000;   // coarsest level at most this many DOFs
-  double ratio = 10.0;     // smoothing interval [lambda/ratio, lambda]
+  // smoothing interval [lambda/ratio, lambda]: 14 in elasticity (10 and 20
+  // gave 16.4 and 15.7 ms per OC iteration at 120x60x60, 8 loads, 14 gave
+  // 15.5; 30 needs up to 150 iterations where the design has just changed)
+  double ratio = 14.0, ratio_scalar = 10.0;
   int power_iters = 20;
 };
 
 // Build the level structure for an operator (no numeric data yet).  Returns
 // false when the grid cannot be coarsened to at most max_coarse DOFs.
 bool mg_plan(const skt_operator* op, const MGConfig& cfg, std::vector<MGLevel>* out);
+
+// Whether factors 2, 3 and 5 that divide the axes reach max_coarse DOFs, the
+// grids that an explicit request for multigrid is documented to take.
+bool mg_divides(const skt_operator* op, const MGConfig& cfg);
 
 // Allocate buffers for dtype and k columns (idempotent for the same dtype).
 int mg_alloc(MGData* mg, const skt_operator* op, const MGConfig& cfg, int dtype, int max_cols);

@@ -1163,6 +1163,7 @@ int skt_hex8_create_scalar(int64_t nx, int64_t ny, int64_t nz, double hx, double
   hex_K0(SKT_HEAT, 0.0, op->h, 2, Kc);
   hex_M0(op->h, M);
   for (int i = 0; i < 64; ++i) op->K0h[i] = mass_coef * M[i] + stiff_coef * Kc[i];
+  op->mass_a = mass_coef;
   return hex8_finish(op, dof_fixed, out);
 }
 

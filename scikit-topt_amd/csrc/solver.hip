@@ -52,7 +52,7 @@ struct skt_solver {
   int used = SKT_PC_JACOBI;  // the one the last solve ran with
   skt::MGConfig mgcfg;
   skt::MGData mg;
-  int mg_possible = -1;      // -1 unknown, 0 no, 1 yes
+  int mg_possible = -1;      // -1 unknown, 0 no, 1 yes, 2 only where not asked for
   // optional per-launch timing of the operator apply (hipEvents on the
   // solve stream, read back at the convergence checks); only chunks that
   // start with every column live are timed, since the apply skips the work
@@ -827,10 +827,18 @@ static int setup_precond(skt_solver* s, const Blk& b, const double* E64, const V
     std::vector<MGLevel> lv;
     const bool grid = (s->op->mesh == SKT_MESH_HEX8 && s->op->modal_ok) ||
                       (s->op->mesh == SKT_MESH_TET4 && s->op->tet_grid);
-    s->mg_possible = (grid && mg_plan(s->op, s->mgcfg, &lv)) ? 1 : 0;
+    // A grid whose axes factors 2, 3 and 5 do not divide far enough takes the
+    // multigrid by SKT_PC_AUTO, but an explicit request for it stays refused.
+    // Operators with a mass term (the Helmholtz filter's) stay with Jacobi
+    // there: their spectrum is narrow, and the set-up would cost more than
+    // the iterations it saves.
+    s->mg_possible = !(grid && mg_plan(s->op, s->mgcfg, &lv)) ? 0
+                     : mg_divides(s->op, s->mgcfg)            ? 1
+                     : s->op->mass_a == 0.0                   ? 2
+                                                              : 0;
   }
   const bool kc_ok = b.kc <= (s->op->ncomp == 3 ? 2 : 4);
-  if (!s->mg_possible || !kc_ok) {
+  if (!s->mg_possible || !kc_ok || (s->precond == SKT_PC_MG && s->mg_possible == 2)) {
     if (s->precond == SKT_PC_MG) {
       set_error("multigrid needs a structured hex8 grid that coarsens below max_coarse DOFs");
       return SKT_EINVAL;
@@ -838,6 +846,12 @@ static int setup_precond(skt_solver* s, const Blk& b, const double* E64, const V
     return SKT_OK;
   }
   int stt = mg_alloc(&s->mg, s->op, s->mgcfg, v.dtype, s->max_cols);
+  if (stt && s->mg_possible == 2) {  // no room for the hierarchy
+    (void)hipGetLastError();
+    mg_free(&s->mg);
+    s->mg_possible = 0;
+    return SKT_OK;
+  }
   if (stt) return stt;
   stt = run_setup<T>(s, E64, v, st);
   if (stt) return stt;
