@@ -1,0 +1,79 @@
+"""The bisection makes the decisions at multipliers whose rates are all at
+rate_min from one evaluation.  Against the oracle, which evaluates each:
+evaluation count, multiplier and densities, for brackets that leave saturation,
+that stay in it to the end or never reach it, and where nothing is skipped."""
+import numpy as np
+import pytest
+
+from oracle import filter as ofilt
+from oracle import oc as ooc
+from oracle import problems as oprob
+
+pytestmark = pytest.mark.gpu
+
+CASES = {
+    # vol_frac, eta, rate_min, l1, l2, tolerance, max_iter, dC
+    "usual": (0.3, 0.5, 0.7, 1e-7, 1e7, 1e-5, 1000, "usual"),
+    "volume-too-large-throughout": (0.01, 0.5, 0.7, 1e-7, 1e7, 1e-5, 1000, "usual"),
+    "volume-too-small-throughout": (0.99, 0.5, 0.7, 1e-7, 1e7, 1e-5, 1000, "usual"),
+    "bracket-below-saturation": (0.3, 0.5, 0.7, 1e-7, 1.5, 1e-5, 1000, "usual"),
+    "eta-one": (0.3, 1.0, 0.9, 1e-7, 1e7, 1e-5, 1000, "usual"),
+    "eta-two": (0.35, 2.0, 0.5, 1e-7, 1e5, 1e-6, 1000, "usual"),
+    "no-lower-rate": (0.3, 0.5, 0.0, 1e-7, 1e7, 1e-5, 1000, "usual"),
+    "stopped-by-count": (0.3, 0.5, 0.7, 1e-7, 1e7, 1e-5, 5, "usual"),
+    "stopped-after-saturation": (0.3, 0.5, 0.7, 1e-7, 1e7, 1e-5, 30, "usual"),
+    "zero-sensitivities": (0.3, 0.5, 0.7, 1e-7, 1e7, 1e-5, 1000, "zero"),
+    "some-of-the-wrong-sign": (0.3, 0.5, 0.7, 1e-7, 1e7, 1e-5, 1000, "sign"),
+    "not-a-number": (0.3, 0.5, 0.7, 1e-7, 1e7, 1e-5, 1000, "nan"),
+    "infinite": (0.3, 0.5, 0.7, 1e-7, 1e7, 1e-5, 1000, "inf"),
+}
+
+
+@pytest.mark.parametrize("form", ["stencil", "tree", "csr"])
+@pytest.mark.parametrize("name", CASES)
+def test_matches_oracle(gpu, name, form, monkeypatch):
+    import torch
+    from sktopt_amd import _lib, mesh as pmesh
+    from sktopt_amd.filters import SpacialFilter
+    vf, eta, rmin, l1, l2, tol, most, which = CASES[name]
+    task = oprob.cantilever(12, 6, 6)
+    mask = task.design_mask.copy()
+    mask[task.dirichlet_elements] = False
+    design = np.nonzero(mask)[0]
+    rng = np.random.default_rng(3)
+    rho = np.ones(task.n_elements)
+    rho[design] = rng.uniform(0.05, 0.9, design.size)
+    dC = -rng.uniform(0.0, 1.0, design.size) ** 3
+    if which == "zero":
+        dC[:] = 0.0
+    elif which == "sign":
+        dC[::50] *= -1.0
+    elif which == "nan":
+        dC[7] = np.nan
+    elif which == "inf":
+        dC[7] = -np.inf
+    vol = task.elements_volume[design]
+    of = ofilt.SpacialFilter(task.centers, 1.5, mask)
+    ref = ooc.bisection_with_physical_volume(
+        dC, rho[design], rho, design, of, 1e-2, 1.0, 0.2, eta, 1e-12, vf, 2.0, 0.5, vol,
+        vol.sum(), rmin, 1.3, max_iter=most, tolerance=tol, l1=l1, l2=l2)
+    monkeypatch.setenv("SKT_OC_TREE", "0" if form == "csr" else "1")
+    if form == "stencil":
+        f = SpacialFilter(pmesh.structured_hex(12, 6, 6), task.elements_volume, 1.5, mask)
+    else:
+        f = SpacialFilter(None, task.elements_volume, 1.5, mask, element_centers=task.centers)
+    f.handle
+    assert f.stencil_active == (form == "stencil")
+    t = lambda v: torch.as_tensor(v, dtype=torch.float64, device="cuda")  # noqa: E731
+    a = [t(rho), t(rho[design]), t(dC), t(vol)]
+    out = torch.empty(design.size, dtype=torch.float64, device="cuda")
+    res = torch.empty(4, dtype=torch.float64, device="cuda")
+    for _ in range(2):  # the second call starts from the first one's workspaces
+        _lib.call("skt_oc_bisect", f.handle, *[x.data_ptr() for x in a], float(vol.sum()), vf, 0.2,
+                  eta, 1e-2, 1.0, rmin, 1.3, 2.0, 0.5, l1, l2, tol, 1e-4, most, out.data_ptr(),
+                  res.data_ptr(), torch.cuda.current_stream().cuda_stream)
+        r = res.cpu().numpy()
+        assert int(r[2]) == ref[3]
+        np.testing.assert_allclose(r[0], ref[0], rtol=1e-12)
+        # sums of a few hundred terms in another order
+        np.testing.assert_allclose(out.cpu().numpy(), ref[2], rtol=1e-12, atol=1e-14)
