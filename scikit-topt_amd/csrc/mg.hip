@@ -1937,24 +1937,35 @@ static int level_apply(MGData* mg, const skt_operator* op, const void* E, int l,
   const int groups = k / kc;
   const T* st = (const T*)v.st;
   // tile-major levels: LDS-tiled kernel of the level's tile shape (x staged
-  // once per tile); node-major: one (node, row, column group) per thread
+  // once per tile); node-major: one (node, row, column group) per thread.
+  // A workgroup takes up to GMT column groups, which read the tile's
+  // coefficients once.  One group per workgroup where there is only one (the
+  // kernel sums all GM groups it is compiled for; one float32 column, a
+  // Chebyshev step: 9.7 to 8.9 us on 50x25x25 elements, 6.2 to 4.7 us on
+  // 25x13x13), or where the tiles with GMT groups are fewer than the CUs
+  // (20x10x10 elements, 8 float32 columns: 72 workgroups, 7.1 us; 288 with one
+  // group each, 5.2 us).  With more workgroups the coefficients' second and
+  // third read costs more: at a limit of 512, 120x60x60 with 8 loads took 15.6
+  // instead of 14.6 ms per OC iteration, 66x36x28 with 3 loads 6.75 instead of
+  // 6.53.
   constexpr int GMT = sizeof(T) == 4 ? 4 : 2;  // <= 62 KB of LDS for NC * KC = 6
+  const TileShape ts = tile_shape(v.layout);
+  const int64_t tiles = v.layout == ST_NODE ? 0 : st_tiles(v.nx, v.ny, v.nz, ts);
   const unsigned gmb = (unsigned)((groups + GMT - 1) / GMT);
+  const bool single = groups == 1 || tiles * gmb < 256;
+  const unsigned gt = (unsigned)(tiles * (single ? groups : gmb));
   const unsigned g = grid_for(v.nn * op->ncomp * groups);
+#define SKT_ST(NC_, KC_, GM_, S_)                                                                \
+  hipLaunchKernelGGL((k_stencil_apply_tiled<T, NC_, KC_, GM_, MODE, S_.x, S_.y, S_.z>), dim3(gt), \
+                     dim3(S_.x * S_.y * S_.z * NC_), 0, s, v.nx, v.ny, v.nz, groups, st, x, y, oa)
 #define SKT_SA(NC_, KC_)                                                                         \
   do {                                                                                           \
     if (v.layout == ST_TILE_BIG) {                                                               \
-      const unsigned gt = (unsigned)(st_tiles(v.nx, v.ny, v.nz, kTileBig) * gmb);                \
-      hipLaunchKernelGGL((k_stencil_apply_tiled<T, NC_, KC_, GMT, MODE, kTileBig.x, kTileBig.y,   \
-                                                kTileBig.z>),                                    \
-                         dim3(gt), dim3(kTileBig.x * kTileBig.y * kTileBig.z * NC_), 0, s, v.nx,  \
-                         v.ny, v.nz, groups, st, x, y, oa);                                      \
+      if (single) SKT_ST(NC_, KC_, 1, kTileBig);                                                 \
+      else SKT_ST(NC_, KC_, GMT, kTileBig);                                                      \
     } else if (v.layout == ST_TILE_SMALL) {                                                      \
-      const unsigned gt = (unsigned)(st_tiles(v.nx, v.ny, v.nz, kTileSmall) * gmb);              \
-      hipLaunchKernelGGL((k_stencil_apply_tiled<T, NC_, KC_, GMT, MODE, kTileSmall.x,             \
-                                                kTileSmall.y, kTileSmall.z>),                    \
-                         dim3(gt), dim3(kTileSmall.x * kTileSmall.y * kTileSmall.z * NC_), 0, s,  \
-                         v.nx, v.ny, v.nz, groups, st, x, y, oa);                                \
+      if (single) SKT_ST(NC_, KC_, 1, kTileSmall);                                               \
+      else SKT_ST(NC_, KC_, GMT, kTileSmall);                                                    \
     } else {                                                                                     \
       hipLaunchKernelGGL((k_stencil_apply<T, NC_, KC_, 1, MODE>), dim3(g), dim3(kBlock), 0, s,    \
                          v.nx, v.ny, v.nz, groups, st, x, y, oa);                                \
@@ -1971,6 +1982,7 @@ static int level_apply(MGData* mg, const skt_operator* op, const void* E, int l,
     else { set_error("unsupported column block"); return SKT_EINVAL; }
   }
 #undef SKT_SA
+#undef SKT_ST
   SKT_LAUNCH_CHECK();
   return SKT_OK;
 }

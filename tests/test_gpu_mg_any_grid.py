@@ -89,3 +89,22 @@ def test_helmholtz_filter_keeps_its_preconditioner(gpu):
     pc, lev = C.c_int(), C.c_int()
     _lib.call("skt_solver_info", f._ops["forward"][1], C.byref(pc), C.byref(lev))
     assert pc.value == _lib.PC_JACOBI
+
+
+@pytest.mark.parametrize("grid", [(32, 16, 16), (96, 34, 34)])
+@pytest.mark.parametrize("loads", [6, 8])
+def test_column_groups_per_workgroup_give_the_same_bits(gpu, grid, loads, monkeypatch):
+    """Coarse stencil applies with one column group per workgroup (few tiles)
+    or several (level of 48 x 17 x 17 elements), the last one partly filled:
+    bit for bit the node-major kernel's, which takes one group per thread."""
+    task = oprob.multiload(*grid, n_loads=loads, seed=7)
+    rho = _densities(task)
+    out = {}
+    for layout in ("node", "small"):
+        monkeypatch.setenv("SKT_MG_STENCIL_LAYOUT", layout)
+        fem = _fem(task, "elastic", "mixed", 1e-8, "auto")
+        U = np.zeros((task.ndof, loads))
+        fem.objectives_multi_load(rho, 3.0, U)
+        out[layout] = U, fem.last_solve["iters"]
+    assert out["node"][1] == out["small"][1]
+    np.testing.assert_array_equal(out["node"][0], out["small"][0])
