@@ -557,15 +557,20 @@ __global__ void k_stencil_dinv(int64_t nx, int64_t ny, int64_t nz, int layout,
   }
 }
 
-// Dense coarsest matrix (fp64, n x n row-major); zero rows become identity.
+// Dense coarsest matrix (fp64, row-major, n rows padded to np with the
+// identity).
 template <int NC>
 __global__ void k_dense_asm(int64_t nx, int64_t ny, int64_t nz, const double* __restrict__ Kel,
-                            double* __restrict__ A) {
+                            int64_t np, double* __restrict__ A) {
   const int64_t nnx = nx + 1, nny = ny + 1;
   const int64_t n = nnx * nny * (nz + 1) * NC;
-  for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < n * n;
+  for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < np * np;
        t += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t r = t / n, c = t % n;
+    const int64_t r = t / np, c = t % np;
+    if (r >= n || c >= n) {
+      A[t] = r == c ? 1.0 : 0.0;
+      continue;
+    }
     const int64_t nr = r / NC, ncn = c / NC;
     const int d = (int)(r % NC), e = (int)(c % NC);
     const int64_t i = nr % nnx, j = (nr / nnx) % nny, k = nr / (nnx * nny);
@@ -574,241 +579,210 @@ __global__ void k_dense_asm(int64_t nx, int64_t ny, int64_t nz, const double* __
     double v = 0.0;
     if (ox >= -1 && ox <= 1 && oy >= -1 && oy <= 1 && oz >= -1 && oz <= 1)
       v = couple<NC>(Kel, nx, ny, nz, i, j, k, (int)ox, (int)oy, (int)oz, d, e);
-    A[t] = v;
+    // a DOF that no free fine DOF depends on gets the identity
+    A[t] = r == c && !(v > 0.0) ? 1.0 : v;
   }
 }
 
-__global__ void k_dense_fix_diag(int64_t n, double* __restrict__ A) {
-  for (int64_t r = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; r < n;
-       r += (int64_t)gridDim.x * blockDim.x)
-    if (!(A[r * n + r] > 0.0)) A[r * n + r] = 1.0;
-}
-
 // ------------------------------------------- blocked Gauss-Jordan inverse
-// In-place inversion of an SPD matrix (no pivoting needed) by pivot blocks B
-// of kGJ rows: with R the remaining indices,
-//   A_BB <- A_BB^-1, A_BR <- A_BB^-1 A_BR, A_RR <- A_RR - A_RB A_BR(new),
-//   A_RB <- -A_RB A_BB^-1.
-// The three off-block updates are LDS-tiled: kTile x kTile tiles for A_RR
-// (the block dimension in two halves), kTileRC-wide strips for A_BR, A_RB.
+// Inversion of an SPD matrix (no pivoting needed) of T x T blocks of kGJ rows,
+// one pivot block per launch: with P the inverse of pivot block A_bb,
+//   A_bb <- P, A_bJ <- P A_bJ, A_Ib <- -A_Ib P, A_IJ <- A_IJ - A_Ib P A_bJ.
+// The launches alternate between two copies of the matrix, so every block of
+// a launch is independent: a workgroup takes one, forms P A_bJ for itself
+// (float64 matrix instructions; the product twice over costs less than a
+// launch of its own) and applies A_Ib to it.  The first workgroup takes the
+// next pivot block, and inverts it in LDS: that chain, the two products and
+// 16 steps of 4 pivots, is what a launch lasts on small matrices.  Before, a
+// step took three launches with LDS-tiled products on the vector unit and one
+// pivot at a time: n = 1188, 61 us of kernels per step, now 33; n = 1782, 85
+// us, now 42.
 constexpr int kGJ = 64;
-constexpr int kTile = 64;
-constexpr int kTileRC = 32;
+constexpr int kGJStride = kGJ + 16;  // LDS row pitch: two rows of 16 lanes on distinct banks
+typedef double gj_vec4 __attribute__((ext_vector_type(4)));
 
-// invert the pivot block (padded with identity), write it to Binv
-// (kGJ x kGJ) and back into A.  Each thread keeps a 4 x 4 block of the
-// matrix in registers; per pivot k the owners of row k and column k publish
-// them through LDS (double-buffered, so one barrier per pivot), and every
-// thread applies a_ij -= a_ik a_kj / a_kk with column k zeroed first and row
-// k replaced afterwards:
-//   row k:            a_kj / a_kk (j != k),  1 / a_kk (j = k)
-//   column k, i != k: -a_ik / a_kk
-// The pivot index inside a thread's 4 x 4 block is a compile-time constant
-// of the unrolled inner loop, so there is no per-element branching.
-__device__ __forceinline__ void gj_block_inv(int64_t n, int64_t b0, int nb,
-                                             double* __restrict__ A,
-                                             double* __restrict__ Binv) {
+// Inverse of the kGJ x kGJ matrix in LDS (row pitch kGJStride) into P.  Each
+// thread keeps a 4 x 4 block in registers; per step the owners of four pivot
+// rows and columns publish them through LDS (double-buffered, one barrier per
+// step), and every thread inverts the 4 x 4 pivot for itself.
+__device__ __forceinline__ void gj_block_inv(const double* sM, double* __restrict__ P) {
   static_assert(kGJ == 64, "4 x 4 register blocks of a 64 x 64 matrix");
-  __shared__ double prow[2][kGJ], pcol[2][kGJ];
+  __shared__ double prow[2][4][kGJ], pcol[2][kGJ][4];
   const int tid = threadIdx.x;
   const int tr = tid / 16, tc = tid % 16;  // rows 4 tr.., columns 4 tc..
   double m[4][4];
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int r = 4 * tr + i, c = 4 * tc + j;
-      m[i][j] = (r < nb && c < nb) ? A[(b0 + r) * n + b0 + c] : (r == c ? 1.0 : 0.0);
-    }
+    for (int j = 0; j < 4; ++j) m[i][j] = sM[(4 * tr + i) * kGJStride + 4 * tc + j];
   for (int kb = 0; kb < kGJ / 4; ++kb) {
-#pragma unroll
-    for (int ki = 0; ki < 4; ++ki) {
-      const int k = 4 * kb + ki, buf = ki & 1;
-      const bool own_row = tr == kb, own_col = tc == kb;
-      if (own_row) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) prow[buf][4 * tc + j] = m[ki][j];
-      }
-      if (own_col) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) pcol[buf][4 * tr + i] = m[i][ki];
-      }
-      __syncthreads();
-      const double ip = 1.0 / pcol[buf][k];
-      double rk[4], ck[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) rk[j] = prow[buf][4 * tc + j] * ip;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) ck[i] = pcol[buf][4 * tr + i];
-      if (own_col) {
-        rk[ki] = ip;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) m[i][ki] = 0.0;
-      }
+    const int buf = kb & 1;
+    const bool own_row = tr == kb, own_col = tc == kb;
+    if (own_row) {
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) m[i][j] -= ck[i] * rk[j];
-      if (own_row) {
+        for (int j = 0; j < 4; ++j) prow[buf][i][4 * tc + j] = m[i][j];
+    }
+    if (own_col) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) m[ki][j] = rk[j];
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) pcol[buf][4 * tr + i][j] = m[i][j];
+    }
+    __syncthreads();
+    double d[4][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) d[i][j] = prow[buf][i][4 * kb + j];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const double ip = 1.0 / d[k][k];
+      d[k][k] = 1.0;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) d[k][j] *= ip;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if (i == k) continue;
+        const double f = d[i][k];
+        d[i][k] = 0.0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) d[i][j] -= f * d[k][j];
+      }
+    }
+    // the pivot rows' new values in this thread's columns
+    double rk[4][4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      double x[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) x[q] = prow[buf][q][4 * tc + j];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        double v = 0.0;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) v += d[i][q] * x[q];
+        rk[i][j] = own_col ? d[i][j] : v;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      double c[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) c[q] = pcol[buf][4 * tr + i][q];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        double v = own_col ? 0.0 : m[i][j];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) v -= c[q] * rk[q][j];
+        m[i][j] = own_row ? rk[i][j] : v;
       }
     }
   }
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int r = 4 * tr + i, c = 4 * tc + j;
-      Binv[r * kGJ + c] = m[i][j];
-      if (r < nb && c < nb) A[(b0 + r) * n + b0 + c] = m[i][j];
-    }
+    for (int j = 0; j < 4; ++j) P[(4 * tr + i) * kGJ + 4 * tc + j] = m[i][j];
 }
 
-__global__ void __launch_bounds__(256) k_gj_block_inv(int64_t n, int64_t b0, int nb,
-                                                       double* __restrict__ A,
-                                                       double* __restrict__ Binv) {
-  gj_block_inv(n, b0, nb, A, Binv);
-}
-
-// A_BR <- Binv A_BR on a strip of kTileRC columns (columns inside the block
-// are left alone).  Binv is the inverse padded with identity and the strip
-// rows past nb are zero, so the products run over all kGJ rows; each thread
-// keeps 8 outputs (one column, rows tid / 32 + 8 m) in flight.
-__global__ void __launch_bounds__(256) k_gj_rows(int64_t n, int64_t b0, int nb,
-                                                  const double* __restrict__ Binv,
-                                                  double* __restrict__ A) {
-  static_assert(kGJ * kTileRC == 8 * 256, "8 outputs per thread");
-  __shared__ double sB[kGJ][kGJ + 1];
-  __shared__ double sX[kGJ][kTileRC + 1];
-  const int tid = threadIdx.x;
-  const int64_t c0 = (int64_t)blockIdx.x * kTileRC;
-  for (int i = tid; i < kGJ * kGJ; i += 256) sB[i / kGJ][i % kGJ] = Binv[i];
-  for (int i = tid; i < kGJ * kTileRC; i += 256) {
-    const int r = i / kTileRC, c = i % kTileRC;
-    sX[r][c] = (r < nb && c0 + c < n) ? A[(b0 + r) * n + c0 + c] : 0.0;
-  }
+// the first pivot block's inverse
+__global__ void __launch_bounds__(256) k_gj_first(int np, const double* __restrict__ A,
+                                                  double* __restrict__ P) {
+  __shared__ double sM[kGJ * kGJStride];
+  for (int i = threadIdx.x; i < kGJ * kGJ; i += 256)
+    sM[(i / kGJ) * kGJStride + i % kGJ] = A[(int64_t)(i / kGJ) * np + i % kGJ];
   __syncthreads();
-  const int c = tid % kTileRC, rb = tid / kTileRC;
-  double acc[8] = {};
-#pragma unroll 8
-  for (int q = 0; q < kGJ; ++q) {
-    const double x = sX[q][c];
-#pragma unroll
-    for (int mm = 0; mm < 8; ++mm) acc[mm] += sB[rb + 8 * mm][q] * x;
-  }
-  const int64_t col = c0 + c;
-  if (col >= n || (col >= b0 && col < b0 + nb)) return;
-#pragma unroll
-  for (int mm = 0; mm < 8; ++mm) {
-    const int r = rb + 8 * mm;
-    if (r < nb) A[(b0 + r) * n + col] = acc[mm];
-  }
+  gj_block_inv(sM, P);
 }
 
-// A_RR <- A_RR - A_RB A_BR on a kTile x kTile tile (rows or columns inside
-// the block are left alone)
-__global__ void __launch_bounds__(256) k_gj_update(int64_t n, int64_t b0, int nb,
-                                                    double* __restrict__ A) {
-  constexpr int kH = kGJ / 2;             // block dimension in two halves
-  __shared__ double sL[kTile][kH + 1];    // A_RB rows of the tile
-  __shared__ double sU[kH][kTile + 1];    // A_BR columns of the tile
+// Step of pivot block b (its inverse in P): A into Aout, the next pivot's
+// inverse into Pn.  Lane l of v_mfma_f64_16x16x4 holds A[l % 16][l / 16],
+// B[l / 16][l % 16] and D[l / 16 + 4 i][l % 16], i < 4; wavefront w takes
+// rows 16 w .. 16 w + 15 of the workgroup's block.
+__global__ void __launch_bounds__(256) k_gj_step(int np, int b, const double* __restrict__ A,
+                                                 const double* __restrict__ P,
+                                                 double* __restrict__ Aout,
+                                                 double* __restrict__ Pn) {
+  __shared__ double sR[kGJ * kGJStride];
+  const int T = np / kGJ;
+  const int first = b + 1 < T ? (b + 1) * (T + 1) : 0;
+  const int id = ((int)blockIdx.x + first) % (T * T);
+  const int I = id / T, J = id % T;
   const int tid = threadIdx.x;
-  const int64_t r0 = (int64_t)blockIdx.y * kTile, c0 = (int64_t)blockIdx.x * kTile;
-  // 4 x 4 outputs per thread: rows tr + 16 a, columns tc + 16 b
-  const int tr = tid / 16, tc = tid % 16;
-  double acc[4][4] = {};
-  for (int h = 0; h < kGJ; h += kH) {
-    for (int i = tid; i < kTile * kH; i += 256) {
-      const int r = i / kH, q = i % kH;
-      sL[r][q] = (r0 + r < n && h + q < nb) ? A[(r0 + r) * n + b0 + h + q] : 0.0;
-    }
-    for (int i = tid; i < kH * kTile; i += 256) {
-      const int q = i / kTile, c = i % kTile;
-      sU[q][c] = (h + q < nb && c0 + c < n) ? A[(b0 + h + q) * n + c0 + c] : 0.0;
-    }
-    __syncthreads();
-    for (int q = 0; q < kH; ++q) {
-      double l[4], u[4];
-#pragma unroll
-      for (int a = 0; a < 4; ++a) l[a] = sL[tr + 16 * a][q];
-#pragma unroll
-      for (int b = 0; b < 4; ++b) u[b] = sU[q][tc + 16 * b];
-#pragma unroll
-      for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int b = 0; b < 4; ++b) acc[a][b] += l[a] * u[b];
-    }
-    __syncthreads();
-  }
-#pragma unroll
-  for (int a = 0; a < 4; ++a) {
-    const int64_t r = r0 + tr + 16 * a;
-    if (r >= n || (r >= b0 && r < b0 + nb)) continue;
-#pragma unroll
-    for (int b = 0; b < 4; ++b) {
-      const int64_t c = c0 + tc + 16 * b;
-      if (c >= n || (c >= b0 && c < b0 + nb)) continue;
-      A[r * n + c] -= acc[a][b];
-    }
-  }
-}
-
-// A_RB <- -A_RB Binv on a strip of kTileRC rows (rows inside the block are
-// left alone); each thread keeps 8 outputs (one column, rows tid / 64 + 4 m)
-// in flight, the products over all kGJ columns as in k_gj_rows.
-__device__ __forceinline__ void gj_cols(int64_t n, int64_t b0, int nb, int strip,
-                                        const double* __restrict__ Binv,
-                                        double* __restrict__ A) {
-  static_assert(kGJ * kTileRC == 8 * 256, "8 outputs per thread");
-  __shared__ double sB[kGJ][kGJ + 1];
-  __shared__ double sX[kTileRC][kGJ + 1];
-  const int tid = threadIdx.x;
-  const int64_t r0 = (int64_t)strip * kTileRC;
-  for (int i = tid; i < kGJ * kGJ; i += 256) sB[i / kGJ][i % kGJ] = Binv[i];
-  for (int i = tid; i < kTileRC * kGJ; i += 256) {
-    const int r = i / kGJ, q = i % kGJ;
-    sX[r][q] = (r0 + r < n && q < nb) ? A[(r0 + r) * n + b0 + q] : 0.0;
-  }
-  __syncthreads();
-  const int c = tid % kGJ, rb = tid / kGJ;
-  double acc[8] = {};
-#pragma unroll 8
-  for (int q = 0; q < kGJ; ++q) {
-    const double b = sB[q][c];
-#pragma unroll
-    for (int mm = 0; mm < 8; ++mm) acc[mm] += sX[rb + 4 * mm][q] * b;
-  }
-  if (c >= nb) return;
-#pragma unroll
-  for (int mm = 0; mm < 8; ++mm) {
-    const int64_t row = r0 + rb + 4 * mm;
-    if (row >= n || (row >= b0 && row < b0 + nb)) continue;
-    A[row * n + b0 + c] = -acc[mm];
-  }
-}
-
-// Column strips of pivot block b0 (Binv) and, in the one extra workgroup,
-// the inversion of the next pivot block b1 (nb1 > 0) into Binv1: that block
-// is final once the trailing update of b0 has run, and neither touches the
-// other's entries or inverse buffer.
-__global__ void __launch_bounds__(256) k_gj_cols_next(int64_t n, int64_t b0, int nb,
-                                                       const double* __restrict__ Binv,
-                                                       int64_t b1, int nb1,
-                                                       double* __restrict__ Binv1,
-                                                       double* __restrict__ A) {
-  if (blockIdx.x + 1 == gridDim.x) {
-    if (nb1 > 0) gj_block_inv(n, b1, nb1, A, Binv1);
+  double* out = Aout + ((int64_t)I * np + J) * kGJ;
+  if (I == b && J == b) {
+    for (int i = tid; i < kGJ * kGJ; i += 256) out[(int64_t)(i / kGJ) * np + i % kGJ] = P[i];
     return;
   }
-  gj_cols(n, b0, nb, blockIdx.x, Binv, A);
+  const int w = tid / kWave, lr = tid % 16, lk = (tid % kWave) / 16;
+  gj_vec4 acc[4];
+  if (J != b) {
+    // P A_bJ
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[j] = gj_vec4{0.0, 0.0, 0.0, 0.0};
+    const double* x = A + ((int64_t)b * np + J) * kGJ + lr;
+    const double* p = P + (16 * w + lr) * kGJ + lk;
+#pragma unroll 8
+    for (int s = 0; s < kGJ / 4; ++s) {
+      const double a = p[4 * s];
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        acc[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, x[(int64_t)(4 * s + lk) * np + 16 * j],
+                                                      acc[j], 0, 0, 0);
+    }
+    if (I != b) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          sR[(16 * w + lk + 4 * i) * kGJStride + 16 * j + lr] = acc[j][i];
+      const double* y = A + ((int64_t)I * np + J) * kGJ + lr;
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          acc[j][i] = y[(int64_t)(16 * w + lk + 4 * i) * np + 16 * j];
+    }
+  } else {
+    for (int i = tid; i < kGJ * kGJ; i += 256) sR[(i / kGJ) * kGJStride + i % kGJ] = P[i];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[j] = gj_vec4{0.0, 0.0, 0.0, 0.0};
+  }
+  if (I != b) {  // uniform over the workgroup
+    __syncthreads();
+    const double* l = A + ((int64_t)I * np + b) * kGJ + (int64_t)(16 * w + lr) * np + lk;
+#pragma unroll 8
+    for (int s = 0; s < kGJ / 4; ++s) {
+      const double a = -l[4 * s];
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        acc[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+            a, sR[(4 * s + lk) * kGJStride + 16 * j + lr], acc[j], 0, 0, 0);
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      out[(int64_t)(16 * w + lk + 4 * i) * np + 16 * j + lr] = acc[j][i];
+  if (blockIdx.x == 0 && b + 1 < T) {
+    __syncthreads();  // every wavefront has read sR
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) sR[(16 * w + lk + 4 * i) * kGJStride + 16 * j + lr] = acc[j][i];
+    __syncthreads();
+    gj_block_inv(sR, Pn);
+  }
 }
 
+// the n x n matrix out of its padded copy
 template <typename T>
-__global__ void k_cast(int64_t n, const double* __restrict__ a, T* __restrict__ b) {
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
+__global__ void k_cast(int64_t n, int64_t np, const double* __restrict__ a, T* __restrict__ b) {
+  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n * n;
        i += (int64_t)gridDim.x * blockDim.x)
-    b[i] = (T)a[i];
+    b[i] = (T)a[(i / n) * np + i % n];
 }
 
 // ------------------------------------------------------------ operators
@@ -1751,6 +1725,8 @@ __global__ void k_cheb_coef(int nlev, int degree, double ratio, double ratio_low
 // Chebyshev steps whose coefficients are kept per level
 static int coef_steps(const MGData* mg) { return mg->degree + kLowSteps; }
 
+static int64_t gj_pad(int64_t n) { return (n + kGJ - 1) / kGJ * kGJ; }
+
 static size_t tsize(int dtype) { return dtype == SKT_F64 ? sizeof(double) : sizeof(float); }
 
 void mg_free(MGData* mg) {
@@ -1890,7 +1866,7 @@ int mg_alloc(MGData* mg, const skt_operator* op, const MGConfig& cfg, int dtype,
     }
   }
   const int64_t nc = lv[L].ndof;
-  SKT_HIP(hipMalloc(&mg->Ad, sizeof(double) * nc * nc));
+  SKT_HIP(hipMalloc(&mg->Ad, sizeof(double) * 2 * gj_pad(nc) * gj_pad(nc)));
   SKT_HIP(hipMalloc(&mg->Ad2, sizeof(double) * 2 * kGJ * kGJ));
   SKT_HIP(hipMalloc(&mg->Ainv, ts * nc * nc));
   SKT_HIP(hipMalloc(&mg->lam, sizeof(double) * (L + 1) * 2));
@@ -2003,26 +1979,33 @@ static int level_cheb(MGData* mg, const skt_operator* op, int l, int k, int kc, 
   return level_apply<T, ST_CHEB>(mg, op, nullptr, l, k, kc, x, xout, s, oa);
 }
 
-// In-place blocked Gauss-Jordan inverse of the coarsest matrix in Ad, on
-// stream g (pivot block inverses alternate between the two halves of Ad2).
+// Blocked Gauss-Jordan inverse of the coarsest matrix in Ad, on stream g; the
+// result is at gj_result (pivot block inverses alternate between the two
+// halves of Ad2).
 static void queue_gj(MGData* mg, hipStream_t g) {
-  const int64_t n = mg->lv.back().ndof;
-  const unsigned tiles = (unsigned)((n + kTile - 1) / kTile);
-  const unsigned strips = (unsigned)((n + kTileRC - 1) / kTileRC);
-  hipLaunchKernelGGL(k_gj_block_inv, dim3(1), dim3(256), 0, g, n, (int64_t)0,
-                     (int)std::min<int64_t>(kGJ, n), mg->Ad, mg->Ad2);
-  int par = 0;
-  for (int64_t b0 = 0; b0 < n; b0 += kGJ, par ^= 1) {
-    const int nb = (int)std::min<int64_t>(kGJ, n - b0);
-    const int64_t b1 = b0 + kGJ;
-    const int nb1 = b1 < n ? (int)std::min<int64_t>(kGJ, n - b1) : 0;
-    double* bi = mg->Ad2 + par * kGJ * kGJ;
-    double* bi1 = mg->Ad2 + (par ^ 1) * kGJ * kGJ;
-    hipLaunchKernelGGL(k_gj_rows, dim3(strips), dim3(256), 0, g, n, b0, nb, bi, mg->Ad);
-    hipLaunchKernelGGL(k_gj_update, dim3(tiles, tiles), dim3(256), 0, g, n, b0, nb, mg->Ad);
-    hipLaunchKernelGGL(k_gj_cols_next, dim3(strips + 1), dim3(256), 0, g, n, b0, nb,
-                       (const double*)bi, b1, nb1, bi1, mg->Ad);
+  const int np = (int)gj_pad(mg->lv.back().ndof), T = np / kGJ;
+  double *in = mg->Ad, *out = mg->Ad + (int64_t)np * np;
+  double *p = mg->Ad2, *pn = mg->Ad2 + kGJ * kGJ;
+  hipLaunchKernelGGL(k_gj_first, dim3(1), dim3(256), 0, g, np, (const double*)in, p);
+  for (int b = 0; b < T; ++b) {
+    hipLaunchKernelGGL(k_gj_step, dim3((unsigned)(T * T)), dim3(256), 0, g, np, b,
+                       (const double*)in, (const double*)p, out, pn);
+    std::swap(in, out);
+    std::swap(p, pn);
   }
+}
+
+static const double* gj_result(const MGData* mg) {
+  const int64_t np = gj_pad(mg->lv.back().ndof);
+  return mg->Ad + (np / kGJ % 2 ? np * np : 0);
+}
+
+// the inverse in the cycle's precision
+template <typename T>
+static void queue_cast(MGData* mg, hipStream_t g) {
+  const int64_t n = mg->lv.back().ndof;
+  hipLaunchKernelGGL(k_cast<T>, dim3(grid_for(n * n)), dim3(kBlock), 0, g, n, gj_pad(n),
+                     gj_result(mg), (T*)mg->Ainv);
 }
 
 bool mg_lagged(const MGData* mg) { return mg->lag && mg->have_inv; }
@@ -2063,14 +2046,9 @@ static void fine_timer_end(MGData* mg, int i, hipStream_t) {
 
 int mg_lag_pre(MGData* mg, hipStream_t s) {
   if (!mg->inv_pending) return SKT_OK;
-  const int64_t n = mg->lv.back().ndof;
   SKT_HIP(hipStreamWaitEvent(s, mg->ev_gj, 0));
-  if (mg->dtype == SKT_F64)
-    hipLaunchKernelGGL(k_cast<double>, dim3(grid_for(n * n)), dim3(kBlock), 0, s, n * n,
-                       (const double*)mg->Ad, (double*)mg->Ainv);
-  else
-    hipLaunchKernelGGL(k_cast<float>, dim3(grid_for(n * n)), dim3(kBlock), 0, s, n * n,
-                       (const double*)mg->Ad, (float*)mg->Ainv);
+  if (mg->dtype == SKT_F64) queue_cast<double>(mg, s);
+  else queue_cast<float>(mg, s);
   SKT_LAUNCH_CHECK();
   mg->inv_pending = 0;
   return SKT_OK;
@@ -2231,17 +2209,16 @@ static int setup_t(MGData* mg, const skt_operator* op, const double* E64, const 
       SKT_HIP(hipEventRecord(mg->ev_join, g));
       return SKT_OK;
     }
+    const int64_t np = gj_pad(n);
     if (NC == 3)
-      hipLaunchKernelGGL((k_dense_asm<3>), dim3(grid_for(n * n)), dim3(kBlock), 0, g, c.nx, c.ny,
-                         c.nz, c.Kel, mg->Ad);
+      hipLaunchKernelGGL((k_dense_asm<3>), dim3(grid_for(np * np)), dim3(kBlock), 0, g, c.nx,
+                         c.ny, c.nz, c.Kel, np, mg->Ad);
     else
-      hipLaunchKernelGGL((k_dense_asm<1>), dim3(grid_for(n * n)), dim3(kBlock), 0, g, c.nx, c.ny,
-                         c.nz, c.Kel, mg->Ad);
-    hipLaunchKernelGGL(k_dense_fix_diag, dim3(grid_for(n)), dim3(kBlock), 0, g, n, mg->Ad);
+      hipLaunchKernelGGL((k_dense_asm<1>), dim3(grid_for(np * np)), dim3(kBlock), 0, g, c.nx,
+                         c.ny, c.nz, c.Kel, np, mg->Ad);
     if (!lagged) {
       queue_gj(mg, g);
-      hipLaunchKernelGGL(k_cast<T>, dim3(grid_for(n * n)), dim3(kBlock), 0, g, n * n, mg->Ad,
-                         (T*)mg->Ainv);
+      queue_cast<T>(mg, g);
     }
     SKT_LAUNCH_CHECK();
     SKT_HIP(hipEventRecord(mg->ev_join, g));

@@ -59,7 +59,7 @@ struct MGData {
   int dtype = -1;                     // SKT_F64 / SKT_F32 the buffers hold
   int max_cols = 0;
   std::vector<MGLevel> lv;            // lv[0]: fine level (vector: x only)
-  double* Ad = nullptr;               // coarsest dense matrix, fp64 (n x n), ping
+  double* Ad = nullptr;               // coarsest dense matrix, fp64, padded: two copies
   double* Ad2 = nullptr;              // inverses of the current and next pivot blocks
   void* Ainv = nullptr;               // coarsest inverse in T
   double* lam = nullptr;              // per level lambda_max(D^-1 A) estimates

@@ -108,3 +108,28 @@ def test_column_groups_per_workgroup_give_the_same_bits(gpu, grid, loads, monkey
         out[layout] = U, fem.last_solve["iters"]
     assert out["node"][1] == out["small"][1]
     np.testing.assert_array_equal(out["node"][0], out["small"][0])
+
+
+@pytest.mark.parametrize("grid,coarse", [((6, 6, 6), 64), ((4, 6, 8), 60), ((8, 8, 6), 100),
+                                         ((10, 6, 8), 120), ((14, 8, 6), 160), ((14, 14, 14), 512),
+                                         ((20, 12, 8), 385)])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_coarsest_inverse_sizes(gpu, grid, coarse, precision):
+    """Two levels whose coarsest matrix has one row less, as many, or a few more
+    than a multiple of the pivot block's 64 rows.  With an exact coarse solve the
+    cycle contracts fast; a wrong inverse would not converge in these counts."""
+    task = oprob.heat_patch(grid[0], patch=3)
+    from oracle import mesh as om
+    task.mesh = om.structured_hex(*grid)
+    task.dirichlet_dofs = np.arange(0, (grid[0] + 1) * (grid[1] + 1), 3)
+    task.dirichlet_nodes = task.dirichlet_dofs
+    task.forces = [np.ones(task.mesh.nnodes)]
+    rho = np.random.default_rng(8).uniform(0.3, 1.0, task.mesh.nelements)
+    ofe = ofem.HeatFEM(task, 1e-3)
+    Uo = np.zeros((task.mesh.nnodes, 1))
+    ofe.objectives_multi_load(rho, 3.0, Uo)
+    fem = _fem(task, "heat", precision, 1e-10, "mg", coarse)
+    U = np.zeros((task.mesh.nnodes, 1))
+    fem.objectives_multi_load(rho, 3.0, U)
+    assert fem.last_solve["levels"] == 2 and fem.last_solve["iters"] <= 24
+    assert np.abs(U - Uo).max() <= 1e-7 * np.abs(Uo).max()
