@@ -385,6 +385,13 @@ int skt_solver_configure(skt_solver* s, int precond, int smooth_degree,
                          int max_coarse);
 int skt_solver_info(const skt_solver* s, int* precond_used, int* levels);
 
+/* fixed = 1: the caller's promise that every solve from here on has the
+ * operator and the moduli (values) of the next one, as the Helmholtz filter's
+ * solves do (filters/helmholtz_filter_nodal.py:140-146, rebuilt per radius).
+ * The diagonal and the preconditioner are then set up by that solve only.
+ * 0 (default): set up by every solve. */
+int skt_solver_fix_moduli(skt_solver* s, int fixed);
+
 /* Measurement hooks (no reference counterpart; used by the benchmark):
  * with timing enabled, every operator apply inside the CG loop is bracketed
  * by hipEvents on the solve stream.  get_timing returns the accumulated

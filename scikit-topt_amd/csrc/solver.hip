@@ -47,6 +47,12 @@ struct skt_solver {
   // inverse has served beyond its own
   int64_t it_last = 0, it_prev = 0;
   int inv_age = 0;
+  // The operator and moduli stay as they are between solves
+  // (skt_solver_fix_moduli): the diagonal and the preconditioner of the first
+  // solve in a mode serve the later ones, as long as their buffers live.
+  int fixed_moduli = 0;
+  int ready_mode = -1, ready_used = 0;
+  uint64_t ready_gen = 0;
   // preconditioner
   int precond = SKT_PC_AUTO;
   int used = SKT_PC_JACOBI;  // the one the last solve ran with
@@ -996,12 +1002,20 @@ int skt_solver_configure(skt_solver* s, int precond, int smooth_degree, int max_
   SKT_CHECK(smooth_degree >= 1 && smooth_degree <= 8, "smooth_degree must be in [1, 8]");
   SKT_CHECK(max_coarse >= 8 && max_coarse <= 6000, "max_coarse must be in [8, 6000]");
   s->precond = precond;
+  s->ready_mode = -1;
   if (s->mgcfg.degree != smooth_degree || s->mgcfg.max_coarse != max_coarse) {
     mg_free(&s->mg);
     s->mg_possible = -1;
   }
   s->mgcfg.degree = smooth_degree;
   s->mgcfg.max_coarse = max_coarse;
+  return SKT_OK;
+}
+
+int skt_solver_fix_moduli(skt_solver* s, int fixed) {
+  SKT_CHECK(s, "null solver");
+  s->fixed_moduli = fixed ? 1 : 0;
+  s->ready_mode = -1;
   return SKT_OK;
 }
 
@@ -1095,24 +1109,34 @@ int skt_solver_solve(skt_solver* s, int mode, int ncols, const double* E64,
                      (const double*)s->f64, s->x64);
   SKT_LAUNCH_CHECK();
   int stt;
+  const bool ready = s->fixed_moduli && s->ready_mode == mode && s->ready_gen == s->mg.gen;
+  if (ready) s->used = s->ready_used;
+  s->ready_mode = -1;  // until this solve's set-up has succeeded
   if (mode == SKT_F64) {
-    stt = op_diag(s->op, SKT_F64, E64, s->q64, st);
-    if (stt) return stt;
-    hipLaunchKernelGGL(k_dinv<double>, dim3(grid_for(n)), dim3(kBlock), 0, st, n, s->q64,
-                       s->op->fixed, s->dinv64);
     Vecs<double> v{s->x64, s->r64, s->p64, s->q64, s->z64, s->dinv64, E64, SKT_F64};
-    if ((stt = setup_precond<double>(s, b, E64, v, st))) return stt;
+    if (!ready) {
+      stt = op_diag(s->op, SKT_F64, E64, s->q64, st);
+      if (stt) return stt;
+      hipLaunchKernelGGL(k_dinv<double>, dim3(grid_for(n)), dim3(kBlock), 0, st, n, s->q64,
+                         s->op->fixed, s->dinv64);
+      if ((stt = setup_precond<double>(s, b, E64, v, st))) return stt;
+    }
     stt = solve_t<double>(s, mode, b, E64, v, rtol, maxiter, inner_rtol, iters, st);
   } else {
-    stt = op_diag(s->op, SKT_F32, E32, s->q32, st);
-    if (stt) return stt;
-    hipLaunchKernelGGL(k_dinv<float>, dim3(grid_for(n)), dim3(kBlock), 0, st, n, s->q32,
-                       s->op->fixed, s->dinv32);
     Vecs<float> v{s->d32, s->r32, s->p32, s->q32, s->z32, s->dinv32, E32, SKT_F32};
-    if ((stt = setup_precond<float>(s, b, E64, v, st))) return stt;
+    if (!ready) {
+      stt = op_diag(s->op, SKT_F32, E32, s->q32, st);
+      if (stt) return stt;
+      hipLaunchKernelGGL(k_dinv<float>, dim3(grid_for(n)), dim3(kBlock), 0, st, n, s->q32,
+                         s->op->fixed, s->dinv32);
+      if ((stt = setup_precond<float>(s, b, E64, v, st))) return stt;
+    }
     stt = solve_t<float>(s, mode, b, E64, v, rtol, maxiter, inner_rtol, iters, st);
   }
   if (stt != SKT_OK && stt != SKT_ENOCONV) return stt;
+  s->ready_mode = mode;
+  s->ready_used = s->used;
+  s->ready_gen = s->mg.gen;
   if (stt == SKT_OK) {
     s->it_prev = s->it_last;
     s->it_last = iters[0];

@@ -62,6 +62,7 @@ SIGNATURES = {
     "skt_solver_create": [_vp, _i32, _pp],
     "skt_solver_destroy": [_vp],
     "skt_solver_configure": [_vp, _i32, _i32, _i32],
+    "skt_solver_fix_moduli": [_vp, _i32],
     "skt_hex8_create_scalar": [_i64, _i64, _i64, _d, _d, _d, _d, _d, _vp, _pp],
     "skt_hex8_elem_to_node": [_i64, _i64, _i64, _i32, _vp, _vp, _d, _vp, _vp, _vp],
     "skt_hex8_node_to_elem": [_i64, _i64, _i64, _i32, _vp, _i32, _i32, _vp, _vp],

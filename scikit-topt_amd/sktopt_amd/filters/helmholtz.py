@@ -131,6 +131,8 @@ class HelmholtzFilterNodal:
         op = self._scalar_op(1.0, self.radius ** 2, fixed)
         s = C.c_void_p()
         _lib.call("skt_solver_create", op, int(ncols), C.byref(s))
+        # unit moduli, one operator per radius: one set-up per solver
+        _lib.call("skt_solver_fix_moduli", s, 1)
         self._ops[case] = (op, s, int(ncols))
         return self._ops[case]
 

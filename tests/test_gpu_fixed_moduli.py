@@ -1,0 +1,50 @@
+"""Solvers told that their moduli stay the same set up once: the later solves
+give what a solver that sets up every time gives, in both modes, after a change
+of mode and after a change of the preconditioner."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("grid", [(20, 16, 14), (23, 19, 13)])  # multigrid, Jacobi
+def test_later_solves_equal_fresh_set_ups(gpu, grid):
+    import torch
+    from sktopt_amd import _lib
+    n = int(np.prod([g + 1 for g in grid]))
+    dev = dict(dtype=torch.float64, device="cuda")
+    fixed = torch.zeros(n, dtype=torch.uint8, device="cuda")
+    E = torch.ones(int(np.prod(grid)), **dev)
+    E32 = E.float()
+    op = C.c_void_p()
+    _lib.call("skt_hex8_create_scalar", *grid, 1.0, 1.0, 1.0, 1.0, 4.0, fixed.data_ptr(),
+              C.byref(op))
+    s = {}
+    for keep in (0, 1):
+        s[keep] = C.c_void_p()
+        _lib.call("skt_solver_create", op, 2, C.byref(s[keep]))
+        _lib.call("skt_solver_fix_moduli", s[keep], keep)
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    for step, mode in enumerate((_lib.F64, _lib.F64, _lib.F32, _lib.F32, _lib.F64, _lib.F64)):
+        if step == 5:
+            for v in s.values():
+                _lib.call("skt_solver_configure", v, _lib.PC_JACOBI, 2, 2000)
+        F = torch.rand((n, 2), generator=gen, **dev)
+        out = {}
+        for keep, v in s.items():
+            U = torch.zeros((n, 2), **dev)
+            it, rr = (C.c_int64 * 2)(), (C.c_double * 2)()
+            _lib.call("skt_solver_solve", v, mode, 2, E.data_ptr(), E32.data_ptr(), F.data_ptr(),
+                      U.data_ptr(), 1e-11, 5000, 0.0, it, rr,
+                      torch.cuda.current_stream().cuda_stream)
+            assert max(rr) <= 1e-11
+            out[keep] = U.cpu().numpy()
+        # the power iteration of a repeated set-up refines the smoother's
+        # bound, so the iterates differ within the residual's tolerance (the
+        # operator's condition number is below 100)
+        assert np.abs(out[1] - out[0]).max() <= 2e-9 * np.abs(out[0]).max()
+    for v in s.values():
+        _lib.load().skt_solver_destroy(v)
+    _lib.load().skt_operator_destroy(op)
