@@ -35,6 +35,9 @@ struct skt_filter {
   int64_t gnx = 0, gny = 0, gnz = 0;
   int n_off = 0;
   int R = 0;                       // stencil half-width in elements
+  int rt[3] = {0, 0, 0};           // the offsets' largest components
+  int32_t* dl = nullptr;           // (n_off) the offsets in the LDS tile
+  double* w_el = nullptr;          // (n_el) inv_rs by element, 0 off the design rows
   int32_t* off = nullptr;          // (n_off) packed dx, dy, dz, ascending element order
   int32_t* del = nullptr;          // (n_off) element-index delta
   double* u_off = nullptr;         // (n_off) unnormalised Gaussian weight
@@ -221,6 +224,38 @@ __global__ void k_transpose_values(int64_t n_design, const int32_t* __restrict__
   }
 }
 
+// Sum of val[q] x[gcol[q]] over a lane's entries q = s0 + sub, s0 + sub + kSeg,
+// ... of a row, in that order.  The columns and weights of kAhead entries are
+// loaded together, then their gathers: one entry at a time, a row of 85 entries
+// was eleven waits for memory twice over (60x30x30 cells of six tets, 27.6M
+// entries: 105 us, 3.2 TB/s of weights and columns; now 71 us, 4.7 TB/s).  Loads past the row's
+// end read its last entry and add nothing.
+constexpr int kAhead = 4;
+__device__ __forceinline__ double csr_row(int64_t s0, int64_t s1, int sub,
+                                          const int32_t* __restrict__ gcol,
+                                          const double* __restrict__ val,
+                                          const double* __restrict__ x) {
+  double acc = 0.0;
+  for (int64_t q = s0 + sub; q < s1; q += kAhead * kSeg) {
+    int32_t c[kAhead];
+    double w[kAhead], xv[kAhead];
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) {
+      const int64_t t = q + i * kSeg < s1 ? q + i * kSeg : s1 - 1;
+      c[i] = gcol[t];
+      w[i] = val[t];
+    }
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) xv[i] = x[c[i]];
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) {
+      const double t = acc + w[i] * xv[i];
+      acc = q + i * kSeg < s1 ? t : acc;
+    }
+  }
+  return acc;
+}
+
 // y[e] = x[e] for non-design e; y[design row] = sum_q val[q] x[gcol[q]].
 // kSeg lanes share one row; fixed butterfly reduction inside the segment.
 __global__ void k_csr_apply(int64_t n_el, const int32_t* __restrict__ colmap,
@@ -235,8 +270,7 @@ __global__ void k_csr_apply(int64_t n_el, const int32_t* __restrict__ colmap,
     const int32_t r = colmap[e];
     double acc = 0.0;
     if (r >= 0) {
-      const int64_t s0 = row_ptr[r], s1 = row_ptr[r + 1];
-      for (int64_t q = s0 + sub; q < s1; q += kSeg) acc += val[q] * x[gcol[q]];
+      acc = csr_row(row_ptr[r], row_ptr[r + 1], sub, gcol, val, x);
     }
 #pragma unroll
     for (int off = kSeg / 2; off > 0; off >>= 1) acc += __shfl_xor(acc, off, kSeg);
@@ -379,6 +413,112 @@ __device__ __forceinline__ double stencil_row(int e, int32_t r, int nx, int ny, 
     }
   }
   return acc;
+}
+
+// The same sums from LDS: a workgroup stages x (zero off the grid and, without
+// kDesignX, off the design rows) of a kTX x kTY x TZ block of elements and its
+// halo, and for the transpose the rows' 1 / row-sum beside it.  An offset is
+// then one LDS read and three float64 operations, in the order of stencil_row;
+// there it is two gathers and a dozen integer operations: 128^3 elements, 33
+// offsets, adjoint 84 to 43 us, forward 50 to 37 us; 75^3 with 93 offsets, both,
+// 112 to 69 us.  One workgroup sums 256 elements, or 512 (two per thread, with
+// one read of the offsets) where that leaves at least two workgroups per CU;
+// 1024 gave 62 us for the adjoint (one workgroup's LDS per CU).
+struct FilterTile {
+  int rx, ry, rz;                  // halo, the offsets' largest components
+  const int32_t* __restrict__ dl;  // (n_off) LDS distance of the neighbour
+  const double* __restrict__ w;    // (n_el) 1 / row-sum, 0 off the design rows
+};
+constexpr int kTX = 32, kTY = 4;
+constexpr size_t kTileLds = 61440;
+
+__host__ __device__ inline int tile_cells(int rx, int ry, int rz, int tz) {
+  return (kTX + 2 * rx) * (kTY + 2 * ry) * (tz + 2 * rz);
+}
+
+template <bool kTranspose, bool kDesignX, int TZ>
+__device__ __forceinline__ void tile_rows(double* sx, int nx, int ny, int nz, FilterTile t,
+                                          int n_off, const double* __restrict__ u,
+                                          const int32_t* __restrict__ colmap,
+                                          const double* __restrict__ x, int (&el)[TZ / 2],
+                                          int32_t (&row)[TZ / 2], double (&acc)[TZ / 2]) {
+  constexpr int M = TZ / 2;  // elements of a thread: planes lz, lz + 2
+  const int hx = kTX + 2 * t.rx, hy = kTY + 2 * t.ry;
+  const int cells = hx * hy * (TZ + 2 * t.rz);
+  double* sw = sx + cells;
+  const int bx = (nx + kTX - 1) / kTX, by = (ny + kTY - 1) / kTY;
+  const int x0 = (int)(blockIdx.x % bx) * kTX, y0 = (int)(blockIdx.x / bx % by) * kTY;
+  const int z0 = (int)(blockIdx.x / (bx * by)) * TZ;
+  // a wavefront stages rows of the block (hx <= kTX + 24 values), four rows'
+  // loads in flight together, unpredicated; the row index is uniform, so its
+  // split and bounds are scalar work
+  const int lane = threadIdx.x % kWave, rows = hy * (TZ + 2 * t.rz);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int gx = x0 - t.rx + lane;
+  const bool inx = gx >= 0 && gx < nx;
+  const int jx = inx ? gx : 0;
+  for (int r0 = wave; r0 < rows; r0 += 4 * (256 / kWave)) {
+    double xv[4], wv[4];
+    bool in[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int r = r0 + k * (256 / kWave);
+      const int gy = y0 - t.ry + r % hy, gz = z0 - t.rz + r / hy;
+      const bool row = gy >= 0 && gy < ny && gz >= 0 && gz < nz;
+      in[k] = inx && row;
+      const int j = (row ? nx * (gy + ny * gz) : 0) + jx;
+      xv[k] = x[j];
+      if constexpr (!kDesignX || kTranspose) wv[k] = t.w[j];
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int r = r0 + k * (256 / kWave);
+      if (r >= rows || lane >= hx) continue;
+      bool ok = in[k];
+      if constexpr (!kDesignX || kTranspose) ok = ok && wv[k] != 0.0;
+      sx[r * hx + lane] = ok ? xv[k] : 0.0;
+      if constexpr (kTranspose) sw[r * hx + lane] = ok ? wv[k] : 0.0;
+    }
+  }
+  __syncthreads();
+  const int lx = threadIdx.x % kTX, ly = threadIdx.x / kTX % kTY, lz = threadIdx.x / (kTX * kTY);
+  const int at = t.rx + lx + hx * (t.ry + ly + hy * (t.rz + lz));
+  double ir[M];
+#pragma unroll
+  for (int m = 0; m < M; ++m) {
+    const int ex = x0 + lx, ey = y0 + ly, ez = z0 + lz + 2 * m;
+    const bool in = ex < nx && ey < ny && ez < nz;
+    el[m] = in ? ex + nx * (ey + ny * ez) : -1;
+    row[m] = in ? colmap[el[m]] : -1;
+    ir[m] = !kTranspose && in ? t.w[el[m]] : 0.0;
+    acc[m] = 0.0;
+  }
+#pragma unroll 4
+  for (int o = 0; o < n_off; ++o) {
+    const double uo = u[o];
+    const int a = at + t.dl[o];
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+      const int b = a + 2 * m * hx * hy;
+      const double w = (kTranspose ? sw[b] : ir[m]) * uo;
+      acc[m] += w * sx[b];
+    }
+  }
+}
+
+template <bool kTranspose, int TZ>
+__global__ void __launch_bounds__(256)
+k_filter_tile(int nx, int ny, int nz, FilterTile t, int n_off, const double* __restrict__ u,
+              const int32_t* __restrict__ colmap, const double* __restrict__ x,
+              double* __restrict__ y) {
+  extern __shared__ double stile[];
+  int el[TZ / 2];
+  int32_t row[TZ / 2];
+  double acc[TZ / 2];
+  tile_rows<kTranspose, false, TZ>(stile, nx, ny, nz, t, n_off, u, colmap, x, el, row, acc);
+#pragma unroll
+  for (int m = 0; m < TZ / 2; ++m)
+    if (el[m] >= 0) y[el[m]] = row[m] >= 0 ? acc[m] : (kTranspose ? 0.0 : x[el[m]]);
 }
 
 template <bool kTranspose>
@@ -546,9 +686,7 @@ __global__ void k_oc_volume(int64_t n_design, const int32_t* __restrict__ ids,
   const int sub = threadIdx.x & (kSeg - 1);
   double vsum = 0.0;
   for (int64_t r = tid / kSeg; r < n_design; r += ((int64_t)gridDim.x * blockDim.x) / kSeg) {
-    const int64_t s0 = row_ptr[r], s1 = row_ptr[r + 1];
-    double acc = 0.0;
-    for (int64_t q = s0 + sub; q < s1; q += kSeg) acc += w[q] * cand_full[gcol[q]];
+    double acc = csr_row(row_ptr[r], row_ptr[r + 1], sub, gcol, w, cand_full);
 #pragma unroll
     for (int off = kSeg / 2; off > 0; off >>= 1) acc += __shfl_xor(acc, off, kSeg);
     if (sub == 0) {
@@ -559,6 +697,31 @@ __global__ void k_oc_volume(int64_t n_design, const int32_t* __restrict__ ids,
     }
   }
   double b = block_sum(vsum, sh);
+  if (threadIdx.x == 0) part[blockIdx.x] = b;
+}
+
+// The same over tiles of the grid (k_filter_tile); x is zero off the design rows
+template <int TZ>
+__global__ void __launch_bounds__(256)
+k_oc_volume_tile(int nx, int ny, int nz, FilterTile t, int n_off, const double* __restrict__ u,
+                 const int32_t* __restrict__ colmap, const double* __restrict__ cand_full, const double* __restrict__ vol, double beta,
+                 double beta_eta, double tbe, double denom, const double* __restrict__ st,
+                 double* __restrict__ part) {
+  extern __shared__ double stile[];
+  __shared__ double sh[kBlock / kWave];
+  if (st[5] != 0.0) return;
+  int el[TZ / 2];
+  int32_t row[TZ / 2];
+  double acc[TZ / 2];
+  tile_rows<false, true, TZ>(stile, nx, ny, nz, t, n_off, u, colmap, cand_full, el, row, acc);
+  double vsum = 0.0;
+#pragma unroll
+  for (int m = 0; m < TZ / 2; ++m) {
+    if (row[m] < 0) continue;
+    const double proj = (tbe + tanh((acc[m] - beta_eta) * beta)) / denom;
+    vsum += proj * vol[row[m]];
+  }
+  const double b = block_sum(vsum, sh);
   if (threadIdx.x == 0) part[blockIdx.x] = b;
 }
 
@@ -761,6 +924,42 @@ static int cub_call(F f, hipStream_t stream) {
   return SKT_OK;
 }
 
+// Element planes per tile of the LDS form, 0 where its halo does not fit: 4
+// (two elements per thread) where that leaves two workgroups per CU, else 2.
+static int tile_planes(const skt_filter* f, bool transpose) {
+  const int64_t xy = ((f->gnx + kTX - 1) / kTX) * ((f->gny + kTY - 1) / kTY);
+  const size_t per = sizeof(double) * (transpose ? 2 : 1);
+  for (int tz : {4, 2}) {
+    if (per * tile_cells(f->rt[0], f->rt[1], f->rt[2], tz) > kTileLds) continue;
+    if (tz == 2 || xy * ((f->gnz + tz - 1) / tz) >= 512) return tz;
+  }
+  return 0;
+}
+
+static int64_t tile_count(const skt_filter* f, int tz) {
+  return ((f->gnx + kTX - 1) / kTX) * ((f->gny + kTY - 1) / kTY) * ((f->gnz + tz - 1) / tz);
+}
+
+template <bool kTranspose>
+static void launch_stencil_filter(const skt_filter* f, const double* x, double* y,
+                                  hipStream_t stream) {
+  const int tz = tile_planes(f, kTranspose);
+  const FilterTile t{f->rt[0], f->rt[1], f->rt[2], f->dl, f->w_el};
+  const size_t lds = sizeof(double) * (kTranspose ? 2 : 1) *
+                     tile_cells(f->rt[0], f->rt[1], f->rt[2], tz);
+#define SKT_FT(TZ_)                                                                              \
+  hipLaunchKernelGGL((k_filter_tile<kTranspose, TZ_>), dim3((unsigned)tile_count(f, TZ_)),       \
+                     dim3(256), lds, stream, (int)f->gnx, (int)f->gny, (int)f->gnz, t, f->n_off, \
+                     f->u_off, f->colmap, x, y)
+  if (tz == 4) SKT_FT(4);
+  else if (tz == 2) SKT_FT(2);
+  else
+    hipLaunchKernelGGL(k_stencil_filter<kTranspose>, dim3(grid_for(f->n_el)), dim3(kBlock), 0,
+                       stream, (int)f->n_el, (int)f->gnx, (int)f->gny, (int)f->gnz, f->R,
+                       f->n_off, f->off, f->del, f->u_off, f->colmap, f->inv_rs, x, y);
+#undef SKT_FT
+}
+
 extern "C" {
 
 int skt_filter_create(int64_t n_el, const double* centers,
@@ -904,6 +1103,10 @@ int skt_filter_set_grid(skt_filter* f, int64_t nx, int64_t ny, int64_t nz, doubl
   (void)hipFree(f->off);
   (void)hipFree(f->del);
   (void)hipFree(f->u_off);
+  (void)hipFree(f->dl);
+  (void)hipFree(f->w_el);
+  f->dl = nullptr;
+  f->w_el = nullptr;
   f->off = nullptr;
   f->del = nullptr;
   f->u_off = nullptr;
@@ -948,6 +1151,22 @@ int skt_filter_set_grid(skt_filter* f, int64_t nx, int64_t ny, int64_t nz, doubl
       }
   f->n_off = (int)hw.size();
   f->R = R;
+  for (int a = 0; a < 3; ++a) {
+    f->rt[a] = 0;
+    for (int32_t pk : ho) f->rt[a] = std::max(f->rt[a], std::abs(((pk >> (8 * a)) & 255) - 64));
+  }
+  std::vector<int32_t> hl;
+  const int lhx = kTX + 2 * f->rt[0], lhy = kTY + 2 * f->rt[1];
+  for (int32_t pk : ho)
+    hl.push_back((pk & 255) - 64 + lhx * (((pk >> 8) & 255) - 64 + lhy * (((pk >> 16) & 255) - 64)));
+  SKT_HIP(hipMalloc(&f->dl, sizeof(int32_t) * hl.size()));
+  SKT_HIP(hipMalloc(&f->w_el, sizeof(double) * f->n_el));
+  hipLaunchKernelGGL(k_fill, dim3(grid_for(f->n_el)), dim3(kBlock), 0, nullptr, f->n_el, 0.0,
+                     f->w_el);
+  hipLaunchKernelGGL(k_scatter_design, dim3(grid_for(f->n_design)), dim3(kBlock), 0, nullptr,
+                     f->n_design, f->design_ids, f->inv_rs, f->w_el);
+  SKT_LAUNCH_CHECK();
+  SKT_HIP(hipMemcpy(f->dl, hl.data(), sizeof(int32_t) * hl.size(), hipMemcpyHostToDevice));
   SKT_HIP(hipMalloc(&f->off, sizeof(int32_t) * ho.size()));
   SKT_HIP(hipMalloc(&f->del, sizeof(int32_t) * hd.size()));
   SKT_HIP(hipMalloc(&f->u_off, sizeof(double) * hw.size()));
@@ -979,6 +1198,8 @@ int skt_filter_destroy(skt_filter* f) {
   (void)hipFree(f->off);
   (void)hipFree(f->del);
   (void)hipFree(f->u_off);
+  (void)hipFree(f->dl);
+  (void)hipFree(f->w_el);
   (void)hipFree(f->cand_full);
   (void)hipFree(f->cand_tree);
   (void)hipFree(f->part_tree);
@@ -1026,9 +1247,7 @@ int skt_filter_forward(skt_filter* f, const double* x, double* y, hipStream_t st
   SKT_CHECK(f && x && y, "null pointer");
   SKT_CHECK(x != y, "filter forward cannot run in place");
   if (f->stencil)
-    hipLaunchKernelGGL(k_stencil_filter<false>, dim3(grid_for(f->n_el)), dim3(kBlock), 0,
-                       stream, (int)f->n_el, (int)f->gnx, (int)f->gny, (int)f->gnz, f->R,
-                       f->n_off, f->off, f->del, f->u_off, f->colmap, f->inv_rs, x, y);
+    launch_stencil_filter<false>(f, x, y, stream);
   else
     hipLaunchKernelGGL(k_csr_apply, dim3(grid_for(f->n_el * kSeg)), dim3(kBlock), 0, stream,
                        f->n_el, f->colmap, f->row_ptr, f->gcol, f->w, x, y, 0);
@@ -1040,9 +1259,7 @@ int skt_filter_gradient(skt_filter* f, const double* v, double* g, hipStream_t s
   SKT_CHECK(f && v && g, "null pointer");
   SKT_CHECK(v != g, "filter gradient cannot run in place");
   if (f->stencil)
-    hipLaunchKernelGGL(k_stencil_filter<true>, dim3(grid_for(f->n_el)), dim3(kBlock), 0,
-                       stream, (int)f->n_el, (int)f->gnx, (int)f->gny, (int)f->gnz, f->R,
-                       f->n_off, f->off, f->del, f->u_off, f->colmap, f->inv_rs, v, g);
+    launch_stencil_filter<true>(f, v, g, stream);
   else
     hipLaunchKernelGGL(k_csr_apply, dim3(grid_for(f->n_el * kSeg)), dim3(kBlock), 0, stream,
                        f->n_el, f->colmap, f->row_ptr, f->gcol, f->wt, v, g, 1);
@@ -1130,7 +1347,15 @@ int skt_oc_bisect(skt_filter* f, const double* rho_full, const double* rho_e,
     return SKT_OK;
   }
   // passes alternate between the two halves of the state
-  const int nbv = (int)(f->stencil ? nbs : nb);
+  const int tz = f->stencil ? tile_planes(f, false) : 0;
+  const bool tiles = tz && tile_count(f, tz) <= kPartMax;
+  const FilterTile ft{f->rt[0], f->rt[1], f->rt[2], f->dl, f->w_el};
+  const size_t lds = sizeof(double) * tile_cells(f->rt[0], f->rt[1], f->rt[2], tz);
+  const int nbv = tiles ? (int)tile_count(f, tz) : (int)(f->stencil ? nbs : nb);
+#define SKT_OV(TZ_)                                                                              \
+  hipLaunchKernelGGL(k_oc_volume_tile<TZ_>, dim3((unsigned)nbv), dim3(256), lds, stream,         \
+                     (int)f->gnx, (int)f->gny, (int)f->gnz, ft, f->n_off, f->u_off, f->colmap,   \
+                     f->cand_full, vol, beta, beta_eta, tbe, denom, cur, f->part)
   double *cur = f->state, *next = f->state + 16;
   for (int s = 0; s < steps; ++s) {
     hipLaunchKernelGGL(k_oc_step, dim3(grid_for(nd, kBlock, 512)), dim3(kBlock), 0, stream, s == 0 ? 1 : 0,
@@ -1138,7 +1363,11 @@ int skt_oc_bisect(skt_filter* f, const double* rho_full, const double* rho_e,
                        next, nd, f->design_ids, rho_e, dC, 1e-12, eta, rate_min, rate_max,
                        move_limit, rho_min, rho_max, f->cand_full, rho_out);
     std::swap(cur, next);
-    if (f->stencil)
+    if (tiles && tz == 4)
+      SKT_OV(4);
+    else if (tiles)
+      SKT_OV(2);
+    else if (f->stencil)
       hipLaunchKernelGGL(k_oc_volume_stencil, dim3(nbs), dim3(kBlock), 0, stream, (int)nd,
                          f->design_ids, (int)f->gnx, (int)f->gny, (int)f->gnz, f->R, f->n_off,
                          f->off, f->del, f->u_off, f->colmap, f->inv_rs, f->cand_full, vol,
@@ -1148,6 +1377,7 @@ int skt_oc_bisect(skt_filter* f, const double* rho_full, const double* rho_e,
                          f->row_ptr, f->gcol, f->w, f->cand_full, vol, beta, beta_eta, tbe,
                          denom, cur, f->part);
   }
+#undef SKT_OV
   hipLaunchKernelGGL(k_oc_result, dim3(1), dim3(kBlock), 0, stream, nbv, (const double*)f->part,
                      vol_sum, vol_frac, vol_tol, tolerance, max_iter, cur, result);
   SKT_LAUNCH_CHECK();
