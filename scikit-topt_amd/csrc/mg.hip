@@ -1698,14 +1698,17 @@ __global__ void k_pow_scale(int64_t n, const double* __restrict__ inv, const T* 
     v[i] = y[i] * s;
 }
 
-// Chebyshev (c1, c2) per step for the interval [beta/ratio, beta],
-// beta = 1.1 * lambda estimate; the last level takes ratio_low
+// Chebyshev (c1, c2) per step for the interval [beta/ratio, beta]; the last
+// level takes ratio_low.  The residual polynomial stays below 1 in magnitude,
+// and the cycle positive definite, up to beta (1 + 1/ratio): beta is chosen so
+// that this is 1.21 times the power iteration's estimate for every ratio.
 __global__ void k_cheb_coef(int nlev, int degree, double ratio, double ratio_low,
                             const double* __restrict__ lam, double* __restrict__ coef) {
   const int l = threadIdx.x;
   if (l >= nlev) return;
-  const double bmax = 1.1 * lam[l];
-  const double amin = bmax / (l > 0 && l == nlev - 1 ? ratio_low : ratio);
+  const double r = l > 0 && l == nlev - 1 ? ratio_low : ratio;
+  const double bmax = 1.21 / (1.0 + 1.0 / r) * lam[l];
+  const double amin = bmax / r;
   const double theta = 0.5 * (bmax + amin), delta = 0.5 * (bmax - amin);
   const double sigma = theta / delta;
   double* c = coef + (size_t)l * 2 * degree;

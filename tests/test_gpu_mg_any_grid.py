@@ -79,16 +79,46 @@ def test_explicit_request_stays_refused(gpu):
         fem.objectives_multi_load(_densities(task), 3.0, np.zeros((task.ndof, 1)))
 
 
-def test_helmholtz_filter_keeps_its_preconditioner(gpu):
-    """A mass-dominated operator on a grid that 2, 3 and 5 do not divide."""
-    from sktopt_amd import _lib, filters, mesh as pmesh
+@pytest.mark.parametrize("keep", [0, 1])
+def test_mass_operator_takes_it_where_one_set_up_serves_all_solves(gpu, keep):
+    """A Helmholtz operator on a grid that 2, 3 and 5 do not divide: Jacobi with
+    a set-up per solve, multigrid with one for all (as the filter asks for)."""
     import ctypes as C
-    m = pmesh.structured_hex(23, 19, 13)
-    f = filters.HelmholtzFilterNodal(m, m.elements_volume(), 1.5)
-    f.forward(np.full(m.nelements, 0.5))
+    import torch
+    from sktopt_amd import _lib
+    n, e = 24 * 20 * 14, 23 * 19 * 13
+    t = dict(dtype=torch.float64, device="cuda")
+    fixed, E, F = torch.zeros(n, dtype=torch.uint8, device="cuda"), torch.ones(e, **t), \
+        torch.rand((n, 1), **t)
+    op, s = C.c_void_p(), C.c_void_p()
+    _lib.call("skt_hex8_create_scalar", 23, 19, 13, 1.0, 1.0, 1.0, 1.0, 4.0, fixed.data_ptr(),
+              C.byref(op))
+    _lib.call("skt_solver_create", op, 1, C.byref(s))
+    _lib.call("skt_solver_fix_moduli", s, keep)
+    U, it, rr = torch.zeros((n, 1), **t), (C.c_int64 * 2)(), (C.c_double * 1)()
+    _lib.call("skt_solver_solve", s, _lib.F64, 1, E.data_ptr(), None, F.data_ptr(), U.data_ptr(),
+              1e-10, 1000, 0.0, it, rr, torch.cuda.current_stream().cuda_stream)
     pc, lev = C.c_int(), C.c_int()
-    _lib.call("skt_solver_info", f._ops["forward"][1], C.byref(pc), C.byref(lev))
-    assert pc.value == _lib.PC_JACOBI
+    _lib.call("skt_solver_info", s, C.byref(pc), C.byref(lev))
+    assert pc.value == (_lib.PC_MG if keep else _lib.PC_JACOBI) and rr[0] <= 1e-10
+    _lib.load().skt_solver_destroy(s)
+    _lib.load().skt_operator_destroy(op)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_a_cycle_that_breaks_down_falls_back_to_jacobi(gpu, precision, monkeypatch):
+    """SKT_MG_RATIO = 900 leaves the smoother next to no margin above its
+    estimate, so the cycle may lose definiteness; a grid that is only halved
+    still gets its solution."""
+    monkeypatch.setenv("SKT_MG_RATIO", "900")
+    task = oprob.multiload(13, 11, 9, n_loads=2, seed=1)
+    rho = np.where(np.random.default_rng(3).uniform(size=task.n_elements) < 0.5, 1.0, 1e-3)
+    fem = _fem(task, "elastic", precision, 1e-10, "auto", 100)
+    Uo = np.zeros((task.ndof, 2))
+    co = ofem.ElasticFEM(task, 1e-9).objectives_multi_load(rho, 3.0, Uo)
+    U = np.zeros((task.ndof, 2))
+    c = fem.objectives_multi_load(rho, 3.0, U)
+    np.testing.assert_allclose(c, co, rtol=1e-7)
 
 
 @pytest.mark.parametrize("grid", [(32, 16, 16), (96, 34, 34)])
