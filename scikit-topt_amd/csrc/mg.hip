@@ -1389,6 +1389,85 @@ k_restrict222(int fnx, int fny, int fnz, int tiles_x, int tiles_y, int zchunks, 
   }
 }
 
+// The same restriction where its tiles leave CUs idle: a thread per coarse node,
+// component and column group gathers its 27 fine nodes straight from memory, all
+// loads unpredicated (clamped addresses, weight zero), with the weights and in
+// the order of k_restrict222 and the two passes, so the result is theirs bit for
+// bit.  One wait for memory in place of one per staged plane: 21x11x11 coarse
+// nodes, 8 float32 columns, 8.8 to 5.0 us, and 8.3 to 5.8 us with w.
+template <typename T, int NC, int KC, bool HASW>
+__global__ void __launch_bounds__(256)
+k_restrict_gather(int fnx, int fny, int fnz, int groups, const T* __restrict__ b,
+                  const T* __restrict__ w, T* __restrict__ bc, const T* __restrict__ dinv_c,
+                  const double* __restrict__ cf, T* __restrict__ x0) {
+  const int fnnx = fnx + 1, fnny = fny + 1, fnnz = fnz + 1;
+  const int cnnx = (fnx + 1) / 2 + 1, cnny = (fny + 1) / 2 + 1, cnnz = (fnz + 1) / 2 + 1;
+  const int64_t fnn = (int64_t)fnnx * fnny * fnnz, cnn = (int64_t)cnnx * cnny * cnnz;
+  const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (t >= cnn * NC * groups) return;
+  const int d = (int)(t % NC);
+  const int64_t cn = t / NC % cnn, g = t / (NC * cnn);
+  const int I = (int)(cn % cnnx), J = (int)(cn / cnnx % cnny), K = (int)(cn / ((int64_t)cnnx * cnny));
+  // weights of the neighbours -1, 0, 1 (0 where there is none)
+  T wx[3], wy[3], wz[3];
+  int ix[3], iy[3], iz[3];
+  auto axis = [](int C, int fn, T(&wt)[3], int(&at)[3]) {
+    wt[0] = C == 0 ? T(0) : 2 * C > fn ? T(1) : T(0.5);
+    wt[1] = 2 * C > fn ? T(0) : T(1);
+    wt[2] = 2 * C + 1 >= fn ? T(0) : T(0.5);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      const int f = 2 * C + k - 1;
+      at[k] = f < 0 ? 0 : f > fn ? fn : f;
+    }
+  };
+  axis(I, fnx, wx, ix);
+  axis(J, fny, wy, iy);
+  axis(K, fnz, wz, iz);
+  const T* bg = b + (g * fnn * NC + d) * KC;
+  const T* wg = HASW ? w + (g * fnn * NC + d) * KC : nullptr;
+  T v[27][KC], r[HASW ? 27 : 1][KC];
+#pragma unroll
+  for (int o = 0; o < 27; ++o) {
+    const int64_t off =
+        (ix[o % 3] + (int64_t)fnnx * (iy[o / 3 % 3] + (int64_t)fnny * iz[o / 9])) * NC * KC;
+    load_node<T, KC, KC>(bg + off, v[o]);
+    if constexpr (HASW) load_node<T, KC, KC>(wg + off, r[o]);
+  }
+  T acc[KC];
+#pragma unroll
+  for (int c = 0; c < KC; ++c) acc[c] = T(0);
+#pragma unroll
+  for (int dz = 0; dz < 3; ++dz) {
+    T s[KC];
+#pragma unroll
+    for (int c = 0; c < KC; ++c) s[c] = T(0);
+#pragma unroll
+    for (int o = 0; o < 9; ++o) {
+      const T wgt = wx[o % 3] * wy[o / 3];
+#pragma unroll
+      for (int c = 0; c < KC; ++c) {
+        const T q = HASW ? v[9 * dz + o][c] - r[HASW ? 9 * dz + o : 0][c] : v[9 * dz + o][c];
+        const T n = s[c] + wgt * q;
+        s[c] = wgt != T(0) ? n : s[c];
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < KC; ++c) {
+      const T n = acc[c] + wz[dz] * s[c];
+      acc[c] = wz[dz] != T(0) ? n : acc[c];
+    }
+  }
+  const int64_t at = ((g * cnn + cn) * NC + d) * KC;
+  store_node<T, KC, KC>(bc + at, acc);
+  if (x0) {
+    const T s = (T)cf[1] * dinv_c[cn * NC + d];
+#pragma unroll
+    for (int c = 0; c < KC; ++c) acc[c] = s * acc[c];
+    store_node<T, KC, KC>(x0 + at, acc);
+  }
+}
+
 // x_f += Z P x_c.  Thread: fine i; row: (j, k, group).  FIX: Dirichlet flags
 // of the fine level (no correction on fixed DOFs).  Every load of a row (the
 // 8 coarse corners, the fine node, its flags) is unpredicated and issued
@@ -2320,6 +2399,12 @@ static bool fused_transfers_enabled() {
 // Fused restriction into level c when every factor is 2 (k_restrict222; b
 // zero at Dirichlet DOFs); with x0, also the first smoothing iterate of c
 // (coefficients cf).  Returns false, launching nothing, otherwise.
+// Largest coarse level (nodes times column groups) that k_restrict_gather
+// takes: 100x50x50 compliance and gradient 9.36 ms without it, 9.24 up to
+// 32768, 9.04 up to 131072 (its fine level too); 120x60x60 with 8 loads, whose
+// fine level has 230,000, 13.9 ms, and 14.1 with it.
+constexpr int64_t kGatherNodes = 131072;
+
 template <typename T, int NC, int KC>
 static bool launch_restrict_fused(const MGLevel& f, const MGLevel& c, int groups, const T* b,
                                   const T* w, T* bc, const double* cf, T* x0, hipStream_t s) {
@@ -2335,6 +2420,16 @@ static bool launch_restrict_fused(const MGLevel& f, const MGLevel& c, int groups
   const int zch = (cnnz + zlen - 1) / zlen;
   const int64_t nblk = per * zch;
   const T* dc = x0 ? (const T*)c.dinv : nullptr;
+  if (c.nn * groups <= kGatherNodes) {
+    const unsigned gg = (unsigned)((c.nn * NC * groups + 255) / 256);
+    if (w)
+      hipLaunchKernelGGL((k_restrict_gather<T, NC, KC, true>), dim3(gg), dim3(256), 0, s,
+                         (int)f.nx, (int)f.ny, (int)f.nz, groups, b, w, bc, dc, cf, x0);
+    else
+      hipLaunchKernelGGL((k_restrict_gather<T, NC, KC, false>), dim3(gg), dim3(256), 0, s,
+                         (int)f.nx, (int)f.ny, (int)f.nz, groups, b, w, bc, dc, cf, x0);
+    return true;
+  }
   if (w)
     hipLaunchKernelGGL((k_restrict222<T, NC, KC, true>), dim3((unsigned)nblk), dim3(256), 0, s,
                        (int)f.nx, (int)f.ny, (int)f.nz, tiles_x, tiles_y, zch, zlen, b, w, bc,
