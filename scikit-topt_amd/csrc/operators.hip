@@ -631,23 +631,25 @@ k_tet_gather(int64_t n_nodes, int64_t ns, int ncols, const int64_t* __restrict__
 // the apply without per-tet staging.  Phase 1, one thread per tet (the tet
 // arrays are read with consecutive lanes on consecutive tets), computes the
 // tet's four corner forces as k_tet_elem_forces does; a workgroup holds 32
-// whole cells, whose six tets add their forces per cell corner in LDS (tets
-// in order s, local nodes in order), and the cells' 8 corner forces are
-// written corner-major, Fc[((col * 8 + corner) * NC + d) * n_cells + cell],
-// so that consecutive cells are consecutive addresses.
+// whole cells and parks the forces in LDS, where a thread per (cell, corner)
+// adds those of the up to six tets that have the corner (tets in order s) and
+// writes them corner-major, Fc[((col * 8 + corner) * NC + d) * n_cells + cell],
+// so that consecutive cells are consecutive addresses.  A tet's nodes come from
+// its cell and its corner code (4 bytes; the connectivity is 16 of the 76 bytes
+// read per tet).  1.5M tets, one float32 column: 30.9 to 23.2 us; before, 32 threads
+// walked their cells' 24 forces one after the other.
 constexpr int kTgCells = 32;
 
 template <typename T, int NC>
 __global__ void __launch_bounds__(6 * kTgCells)
-k_tetg_cell_forces(int64_t n_cells, int ncols, T lam0, T mu0, T ma, T cb,
-                   const int32_t* __restrict__ code, const int32_t* __restrict__ conn,
-                   const T* __restrict__ g, const T* __restrict__ vol,
+k_tetg_cell_forces(int64_t n_cells, int nx, int ny, int ncols, T lam0, T mu0, T ma, T cb,
+                   const int32_t* __restrict__ code, const T* __restrict__ g,
+                   const T* __restrict__ vol,
                    const T* __restrict__ E, const T* __restrict__ R,
                    const T* __restrict__ X, T* __restrict__ Fc) {
   constexpr int kT = 6 * kTgCells;
   __shared__ T sf[kT][4 * NC + 1];
   __shared__ int scode[kT];
-  __shared__ T sacc[kTgCells][8 * NC];
   const int col = blockIdx.y;
   const int64_t n_el = 6 * n_cells;
   const int tid = threadIdx.x;
@@ -665,9 +667,15 @@ k_tetg_cell_forces(int64_t n_cells, int ncols, T lam0, T mu0, T ma, T cb,
     for (int b = 0; b < 4; ++b)
 #pragma unroll
       for (int d = 0; d < 3; ++d) gg[b][d] = g[(3 * b + d) * n_el + e];
+    // a grid's nodes and cells fit in 32 bits (the connectivity's type)
+    const int cell = (int)(e / 6), ci = cell % nx, cj = cell / nx % ny, ck = cell / (nx * ny);
     int64_t nb[4];
 #pragma unroll
-    for (int b = 0; b < 4; ++b) nb[b] = conn[b * n_el + e];
+    for (int b = 0; b < 4; ++b) {
+      const int c8 = cd >> (3 * b);
+      nb[b] = ci + (c8 & 1) + (int64_t)(nx + 1) * (cj + ((c8 >> 1) & 1) +
+                                                   (int64_t)(ny + 1) * (ck + ((c8 >> 2) & 1)));
+    }
     const T w = E[e] * vol[e];
     if (NC == 1) {
       T x[4];
@@ -725,26 +733,30 @@ k_tetg_cell_forces(int64_t n_cells, int ncols, T lam0, T mu0, T ma, T cb,
 #pragma unroll
     for (int d = 0; d < NC; ++d) sf[tid][a * NC + d] = f[a][d];
   scode[tid] = cd;
-  for (int i = tid; i < kTgCells * 8 * NC; i += kT) sacc[i / (8 * NC)][i % (8 * NC)] = T(0);
-  __syncthreads();
-  if (tid < kTgCells) {
-    for (int s = 0; s < 6; ++s) {
-      const int t = 6 * tid + s;
-      const int c4 = scode[t];
-#pragma unroll
-      for (int a = 0; a < 4; ++a) {
-        const int corner = (c4 >> (3 * a)) & 7;
-#pragma unroll
-        for (int d = 0; d < NC; ++d) sacc[tid][corner * NC + d] += sf[t][a * NC + d];
-      }
-    }
-  }
   __syncthreads();
   const int64_t cell0 = (int64_t)blockIdx.x * kTgCells;
-  for (int i = tid; i < kTgCells * 8 * NC; i += kT) {
-    const int cl = i % kTgCells, v = i / kTgCells;  // v = corner * NC + d
-    if (cell0 + cl < n_cells)
-      Fc[((int64_t)col * 8 * NC + v) * n_cells + cell0 + cl] = sacc[cl][v];
+  for (int i = tid; i < kTgCells * 8; i += kT) {
+    const int cl = i % kTgCells, corner = i / kTgCells;
+    T acc[NC];
+#pragma unroll
+    for (int d = 0; d < NC; ++d) acc[d] = T(0);
+#pragma unroll
+    for (int s = 0; s < 6; ++s) {
+      const int t = 6 * cl + s, c4 = scode[t];
+      int at = -1;  // the corners of a tet are distinct
+#pragma unroll
+      for (int a = 0; a < 4; ++a) at = ((c4 >> (3 * a)) & 7) == corner ? a : at;
+#pragma unroll
+      for (int d = 0; d < NC; ++d) {
+        const T v = acc[d] + sf[t][(at < 0 ? 0 : at) * NC + d];
+        acc[d] = at < 0 ? acc[d] : v;
+      }
+    }
+    if (cell0 + cl < n_cells) {
+#pragma unroll
+      for (int d = 0; d < NC; ++d)
+        Fc[((int64_t)(col * 8 + corner) * NC + d) * n_cells + cell0 + cl] = acc[d];
+    }
   }
 }
 
@@ -930,14 +942,14 @@ static int tet_apply_t(skt_operator* op, int ncols, const T* g, const T* vol, co
     const dim3 g2(std::min<unsigned>(grid_for(op->n_nodes), 65535u), (unsigned)ncols);
     if (op->ncomp == 3) {
       hipLaunchKernelGGL((k_tetg_cell_forces<T, 3>), g1, dim3(6 * kTgCells), 0, s, n_cells,
-                         ncols, (T)op->lam0, (T)op->mu0, (T)op->mass_a, (T)op->cond_b,
-                         op->tet_code, op->conn, g, vol, E, R, X, F);
+                         (int)op->nx, (int)op->ny, ncols, (T)op->lam0, (T)op->mu0,
+                         (T)op->mass_a, (T)op->cond_b, op->tet_code, g, vol, E, R, X, F);
       hipLaunchKernelGGL((k_tetg_gather<T, 3>), g2, dim3(kBlock), 0, s, op->nx, op->ny, op->nz,
                          ncols, (const T*)F, X, op->fixed, Y);
     } else {
       hipLaunchKernelGGL((k_tetg_cell_forces<T, 1>), g1, dim3(6 * kTgCells), 0, s, n_cells,
-                         ncols, (T)op->lam0, (T)op->mu0, (T)op->mass_a, (T)op->cond_b,
-                         op->tet_code, op->conn, g, vol, E, R, X, F);
+                         (int)op->nx, (int)op->ny, ncols, (T)op->lam0, (T)op->mu0,
+                         (T)op->mass_a, (T)op->cond_b, op->tet_code, g, vol, E, R, X, F);
       hipLaunchKernelGGL((k_tetg_gather<T, 1>), g2, dim3(kBlock), 0, s, op->nx, op->ny, op->nz,
                          ncols, (const T*)F, X, op->fixed, Y);
     }
