@@ -40,7 +40,7 @@ struct skt_solver {
          *z64 = nullptr, *dinv64 = nullptr;
   float *r32 = nullptr, *p32 = nullptr, *q32 = nullptr, *z32 = nullptr, *d32 = nullptr,
         *dinv32 = nullptr;
-  double* part = nullptr;   // 4 * kParts * max_cols: area0 | area1
+  double* part = nullptr;   // 2 * kArea * max_cols: area0 | area1
   double* sc = nullptr;     // max_cols * kSc
   double* host = nullptr;   // pinned copy of sc
   // iterations of the last two solves, and set-ups the current coarsest
@@ -106,6 +106,12 @@ struct skt_solver {
 namespace skt {
 
 constexpr int kParts = 512;
+// Partials per column that each of the two areas holds: two quantities of a
+// reduction's kParts blocks, or the workgroups of a modal launch that leaves
+// its product's partials (1053 on 128^3 nodes, 1274 at 200x100x100; beyond it a
+// separate product reads both vectors again, 9 us at 128^3 against one wavefront
+// summing a few more partials).
+constexpr int kArea = 4096;
 constexpr int kSc = 16;
 static_assert(kSc == kStopStride, "the column stop flags are the solver's scalar blocks");
 constexpr int kCheckJacobi = 32;
@@ -587,7 +593,7 @@ static int precondition(skt_solver* s, const Blk& b, const Vecs<T>& v, double* a
   if (s->used == SKT_PC_MG) {
     int slots = 0;
     int stt = mg_vcycle(&s->mg, s->op, v.E, v.dinv, b.k, b.kc, v.r, v.z, v.q, st, fused,
-                        2 * kParts, &slots, stop);
+                        kArea, &slots, stop);
     if (stt) return stt;
     if (slots > 0) {
       *rz_part = fused;
@@ -613,7 +619,7 @@ static int pcg_iterations(skt_solver* s, const Blk& b, const Vecs<T>& v, int64_t
   // area0 (s->part) takes the p.q partials and k_update's r.z / r.r; the
   // fused r.z of the V-cycle goes to area1, which is idle between the
   // initialisation and the reliable updates
-  double* area1 = s->part + (size_t)2 * kParts * s->max_cols;
+  double* area1 = s->part + (size_t)kArea * s->max_cols;
   s->timed = s->timing && !any_flag(s, b.k, S_CONV);
   // a modal operator's apply is timed by its own dispatch (the events
   // bracket the kernel, not the queue around it); others by event records
@@ -625,7 +631,7 @@ static int pcg_iterations(skt_solver* s, const Blk& b, const Vecs<T>& v, int64_t
     }
     int pq_nb = 0;
     // stopped columns' q is not used (alpha = 0), so their work may be skipped
-    int stt = op_apply_dot(s->op, v.dtype, b.k, b.kc, v.E, v.p, v.q, s->part, 2 * kParts,
+    int stt = op_apply_dot(s->op, v.dtype, b.k, b.kc, v.E, v.p, v.q, s->part, kArea,
                            &pq_nb, st, s->sc + S_CONV);
     if (stt) return stt;
     if (s->timed) {
@@ -874,7 +880,7 @@ static int solve_t(skt_solver* s, int mode, const Blk& b, const double* E64, con
   const bool mg = s->used == SKT_PC_MG;
   const int64_t total = b.n * b.k;
   const unsigned ge = grid_for(total);
-  double* area1 = s->part + (size_t)2 * kParts * s->max_cols;
+  double* area1 = s->part + (size_t)kArea * s->max_cols;
   const int check = mg ? mg_poll_interval() : kCheckJacobi;
   // true residual of the initial guess (float64 operator)
   int stt = op_apply(s->op, SKT_F64, b.k, b.kc, E64, s->x64, s->q64, st);
@@ -986,7 +992,7 @@ int skt_solver_create(skt_operator* op, int max_cols, skt_solver** out) {
     SKT_HIP(hipMalloc(p, sizeof(float) * nv));
   SKT_HIP(hipMalloc(&s->dinv64, sizeof(double) * s->n));
   SKT_HIP(hipMalloc(&s->dinv32, sizeof(float) * s->n));
-  SKT_HIP(hipMalloc(&s->part, sizeof(double) * kParts * 4 * max_cols));
+  SKT_HIP(hipMalloc(&s->part, sizeof(double) * 2 * kArea * max_cols));
   SKT_HIP(hipMalloc(&s->sc, sizeof(double) * kSc * max_cols));
   SKT_HIP(hipHostMalloc(&s->host, sizeof(double) * kSc * max_cols, hipHostMallocDefault));
   SKT_HIP(hipEventCreateWithFlags(&s->poll_ev, hipEventDisableTiming));
