@@ -44,7 +44,7 @@ struct skt_filter {
   // bisection workspace
   double* cand_full = nullptr;     // (n_el)
   double* cand_tree = nullptr;     // (n_el, kTreeStride): candidates at the tree's midpoints
-  double* part_tree = nullptr;     // (kTreeK, kPartMax)
+  double* part_tree = nullptr;     // (kTreeStride, kPartMax)
   double* part = nullptr;          // (kPartMax)
   double* state = nullptr;         // bisection state
 };
@@ -58,6 +58,15 @@ constexpr int kTreeLevels = 3;
 constexpr int kTreeK = (1 << kTreeLevels) - 1;
 constexpr int kTreeStride = 8;
 static_assert(kTreeK <= kTreeStride, "tree candidates per element");
+// From this many entries on, a pass evaluates the midpoints that the bisection
+// is expected to meet, kTreeStride of them (oc_path).  A pass is bound by the
+// gather of 64 B per entry: 0.92 ms on 100 x 50 x 50 tets, where an iteration's
+// bisection took 6 to 7 passes over trees (4.9 ms) and takes 2 or 3 along paths
+// (2.6 ms).  The host has to queue a pass for every two evaluations instead of
+// every three, 8 passes more at 46 evaluations, whose launches find the work
+// done and take 5 us each: below 2^22 entries, 30 us a pass, they are not won
+// back.
+constexpr int64_t kPathEntries = (int64_t)1 << 22;
 constexpr int kSeg = 8;  // lanes per CSR row in the gathers
 
 __device__ __forceinline__ double dist2(const double* __restrict__ c, int64_t n,
@@ -587,6 +596,9 @@ __global__ void k_oc_init(int nb, const double* __restrict__ part, double inv_ra
   st[6] = 0.0;
   st[7] = 0.0;
   st[8] = inv_rate < kNoSaturation ? m * inv_rate : kNoSaturation;
+  st[9] = st[10] = nan("");  // volume errors at l1, l2 (k_oc_bracket_tree)
+  st[11] = 1.0;              // the next pass follows a path ...
+  st[12] = l1;               // ... to this multiplier
 }
 
 // One evaluation of the bisection at st[2] with volume error vol_error
@@ -775,6 +787,34 @@ __device__ __forceinline__ void oc_tree(double l1, double l2, double* mid) {
   }
 }
 
+// The midpoints that the bisection of (l1, l2) evaluates on its way to `root`:
+// of those from `sat` on, whose rates are all at rate_min, the first alone
+__device__ __forceinline__ void oc_path(double l1, double l2, double root, double sat,
+                                        double* mid) {
+  for (int n = 0; n < kTreeStride; ++n) {
+    mid[n] = 0.5 * (l1 + l2);
+    if (mid[n] < root) {
+      l1 = mid[n];
+      continue;
+    }
+    l2 = mid[n];
+    if (l2 >= sat)
+      for (int i = 0; i < 128 && 0.5 * (l1 + l2) >= sat; ++i) l2 = 0.5 * (l1 + l2);
+  }
+}
+
+// the K midpoints of a pass: the tree's, or (K = kTreeStride) a path's
+template <int K>
+__device__ __forceinline__ void oc_points(const double* __restrict__ st, double* mid) {
+  if (K == kTreeStride && st[11] != 0.0) {
+    oc_path(st[0], st[1], st[12], st[8], mid);
+    return;
+  }
+  oc_tree(st[0], st[1], mid);
+  if (K > kTreeK) mid[K - 1] = mid[0];
+}
+
+template <int K>
 __global__ void k_oc_candidate_tree(int64_t n_design, const int32_t* __restrict__ ids,
                                     const double* __restrict__ rho_e,
                                     const double* __restrict__ dC,
@@ -783,20 +823,21 @@ __global__ void k_oc_candidate_tree(int64_t n_design, const int32_t* __restrict_
                                     double rho_min, double rho_max,
                                     double* __restrict__ cand_tree) {
   if (st[5] != 0.0) return;
-  double mid[kTreeK];
-  oc_tree(st[0], st[1], mid);
+  double mid[K];
+  oc_points<K>(st, mid);
   for (int64_t r = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; r < n_design;
        r += (int64_t)gridDim.x * blockDim.x) {
     double* out = cand_tree + (int64_t)ids[r] * kTreeStride;
 #pragma unroll
-    for (int k = 0; k < kTreeK; ++k)
+    for (int k = 0; k < K; ++k)
       out[k] = oc_candidate(dC[r], rho_e[r], mid[k], eps, eta, rate_min, rate_max, move_limit,
                             rho_min, rho_max);
   }
 }
 
-// k_oc_volume at every midpoint of the tree: one read of the matrix, the
+// k_oc_volume at every midpoint of the pass: one read of the matrix, the
 // same per-row and per-block summation order for each midpoint.
+template <int K>
 __global__ void k_oc_volume_tree(int64_t n_design, const int64_t* __restrict__ row_ptr,
                                  const int32_t* __restrict__ gcol,
                                  const double* __restrict__ w,
@@ -808,27 +849,27 @@ __global__ void k_oc_volume_tree(int64_t n_design, const int64_t* __restrict__ r
   if (st[5] != 0.0) return;
   const int64_t tid = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   const int sub = threadIdx.x & (kSeg - 1);
-  double vsum[kTreeK];
+  double vsum[K];
 #pragma unroll
-  for (int k = 0; k < kTreeK; ++k) vsum[k] = 0.0;
+  for (int k = 0; k < K; ++k) vsum[k] = 0.0;
   for (int64_t r = tid / kSeg; r < n_design; r += ((int64_t)gridDim.x * blockDim.x) / kSeg) {
     const int64_t s0 = row_ptr[r], s1 = row_ptr[r + 1];
-    double acc[kTreeK];
+    double acc[K];
 #pragma unroll
-    for (int k = 0; k < kTreeK; ++k) acc[k] = 0.0;
+    for (int k = 0; k < K; ++k) acc[k] = 0.0;
     for (int64_t q = s0 + sub; q < s1; q += kSeg) {
       const double wq = w[q];
       const double* c = cand_tree + (int64_t)gcol[q] * kTreeStride;
 #pragma unroll
-      for (int k = 0; k < kTreeK; ++k) acc[k] += wq * c[k];
+      for (int k = 0; k < K; ++k) acc[k] += wq * c[k];
     }
 #pragma unroll
-    for (int k = 0; k < kTreeK; ++k)
+    for (int k = 0; k < K; ++k)
 #pragma unroll
       for (int off = kSeg / 2; off > 0; off >>= 1) acc[k] += __shfl_xor(acc[k], off, kSeg);
     if (sub == 0) {
 #pragma unroll
-      for (int k = 0; k < kTreeK; ++k) {
+      for (int k = 0; k < K; ++k) {
         double t = (acc[k] - beta_eta) * beta;
         t = tanh(t);
         double proj = (tbe + t) / denom;
@@ -836,40 +877,75 @@ __global__ void k_oc_volume_tree(int64_t n_design, const int64_t* __restrict__ r
       }
     }
   }
-  for (int k = 0; k < kTreeK; ++k) {
+  for (int k = 0; k < K; ++k) {
     const double b = block_sum(vsum[k], sh);
     if (threadIdx.x == 0) part[(int64_t)k * gridDim.x + blockIdx.x] = b;
     __syncthreads();
   }
 }
 
-// Walk the tree's path as the sequential bisection would (oc_bracket per
-// level), stopping when it terminates or after max_evals evaluations in all;
-// st[7] keeps the last evaluated midpoint.
+// Take the decisions of a pass as the sequential bisection would (oc_bracket
+// per level), stopping when it terminates, after max_evals evaluations in all,
+// or (path) at a midpoint that was not evaluated because a decision was not
+// the expected one; st[7] keeps the last evaluated midpoint.
+//
+// The next pass: while no volume was too large yet, the path to l1.  Where the
+// volume error is known at both ends, the path to its zero, interpolated in
+// multiplier^-eta, in which the densities are linear as long as no limit holds
+// them: its error shrinks with the bracket, so each path decides more levels
+// than the last.  A path that decided fewer than kTreeLevels is followed by a
+// tree, so that two passes decide four levels or more.
+template <int K>
 __global__ void k_oc_bracket_tree(int nb, const double* __restrict__ part, double vol_sum,
                                   double vol_frac, double vol_tol, double tolerance,
-                                  int max_iter, int max_evals, double* __restrict__ st) {
+                                  int max_iter, int max_evals, double eta,
+                                  double* __restrict__ st) {
   __shared__ double sh[kBlock / kWave];
-  __shared__ double tot[kTreeK];
   if (st[5] != 0.0) return;
-  for (int k = 0; k < kTreeK; ++k) {
-    double v = 0.0;
-    for (int i = threadIdx.x; i < nb; i += blockDim.x) v += part[(int64_t)k * nb + i];
-    const double t = block_sum(v, sh);
-    if (threadIdx.x == 0) tot[k] = t;
+  double v[K], tot[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) v[k] = 0.0;
+  for (int i = threadIdx.x; i < nb; i += blockDim.x)
+#pragma unroll
+    for (int k = 0; k < K; ++k) v[k] += part[(int64_t)k * nb + i];
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    tot[k] = block_sum(v[k], sh);
     __syncthreads();
   }
-  if (threadIdx.x == 0) {
-    double mid[kTreeK];
-    oc_tree(st[0], st[1], mid);
-    int node = 0;
-    for (int lev = 0; lev < kTreeLevels && st[5] == 0.0 && st[6] < (double)max_evals; ++lev) {
-      const double vol_error = tot[node] / vol_sum - vol_frac;
-      oc_bracket(st, vol_error, vol_tol, tolerance, max_iter);
-      node = 2 * node + (vol_error > 0 ? 2 : 1);
-    }
-    oc_saturated(st, vol_tol, tolerance, max_iter, max_evals);
+  if (threadIdx.x) return;
+  __shared__ double vt[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) vt[k] = tot[k];
+  const bool path = K == kTreeStride && st[11] != 0.0;
+  __shared__ double mid[K];
+  if (path) oc_path(st[0], st[1], st[12], st[8], mid);
+  int node = 0, lev = 0;
+  while (lev < (path ? K : kTreeLevels) && st[5] == 0.0 && st[6] < (double)max_evals) {
+    if (path && lev > 0 && st[2] != mid[lev]) break;
+    const double vol_error = vt[node] / vol_sum - vol_frac;
+    oc_bracket(st, vol_error, vol_tol, tolerance, max_iter);
+    st[vol_error > 0 ? 9 : 10] = vol_error;
+    ++lev;
+    node = path ? lev : 2 * node + (vol_error > 0 ? 2 : 1);
+    if (path) oc_saturated(st, vol_tol, tolerance, max_iter, max_evals);
   }
+  if (!path) oc_saturated(st, vol_tol, tolerance, max_iter, max_evals);
+  if (K != kTreeStride) return;
+  st[11] = 0.0;
+  if (path && lev < kTreeLevels) return;
+  const double e1 = st[9], e2 = st[10];
+  if (!(e1 > 0.0)) {
+    st[11] = 1.0;
+    st[12] = st[0];
+    return;
+  }
+  if (!(e2 < 0.0 && st[0] > 0.0 && st[1] < st[8])) return;
+  const double x1 = pow(st[0], -eta), x2 = pow(st[1], -eta);
+  const double r = pow(x1 + (x2 - x1) * (e1 / (e1 - e2)), -1.0 / eta);
+  if (!(r > st[0] && r < st[1])) return;
+  st[12] = r;
+  st[11] = 1.0;
 }
 
 // the design rows' candidate at the last evaluated midpoint (st[7])
@@ -1069,7 +1145,7 @@ int skt_filter_create(int64_t n_el, const double* centers,
   SKT_LAUNCH_CHECK();
   SKT_HIP(hipMalloc(&f->cand_full, sizeof(double) * n_el));
   SKT_HIP(hipMalloc(&f->cand_tree, sizeof(double) * kTreeStride * n_el));
-  SKT_HIP(hipMalloc(&f->part_tree, sizeof(double) * kTreeK * kPartMax));
+  SKT_HIP(hipMalloc(&f->part_tree, sizeof(double) * kTreeStride * kPartMax));
   SKT_HIP(hipMalloc(&f->part, sizeof(double) * kPartMax));
   SKT_HIP(hipMalloc(&f->state, sizeof(double) * 32));
   // the bisection writes the design rows only
@@ -1322,22 +1398,34 @@ int skt_oc_bisect(skt_filter* f, const double* rho_full, const double* rho_e,
   hipLaunchKernelGGL(k_oc_init, dim3(1), dim3(kBlock), 0, stream, (int)nba, f->part, inv_rate,
                      f->state, l1, l2);
   if (!f->stencil && f->cand_tree && oc_tree_enabled()) {
-    // CSR form: kTreeLevels bisection steps per read of the matrix; the
-    // decisions, evaluation count and result equal the step-by-step loop's.
+    // CSR form: kTreeLevels bisection steps per read of the matrix, or up to
+    // kTreeStride along a path; the decisions, evaluation count and result
+    // equal the step-by-step loop's.
     // (The stencil form stays one midpoint per pass: its volume kernel reads
     // no matrix, and seven candidates per offset cost more than the launches
     // they save.)
-    for (int s = 0; s < steps; s += kTreeLevels) {
-      hipLaunchKernelGGL(k_oc_candidate_tree, dim3(grid_for(nd)), dim3(kBlock), 0, stream, nd,
-                         f->design_ids, rho_e, dC, f->state, 1e-12, eta, rate_min, rate_max,
-                         move_limit, rho_min, rho_max, f->cand_tree);
-      hipLaunchKernelGGL(k_oc_volume_tree, dim3(nb), dim3(kBlock), 0, stream, nd, f->row_ptr,
-                         f->gcol, f->w, f->cand_tree, vol, beta, beta_eta, tbe, denom, f->state,
-                         f->part_tree);
-      hipLaunchKernelGGL(k_oc_bracket_tree, dim3(1), dim3(kBlock), 0, stream, (int)nb,
-                         f->part_tree, vol_sum, vol_frac, vol_tol, tolerance, max_iter, steps,
-                         f->state);
+    const bool path = f->nnz >= kPathEntries;
+    // two passes along paths decide at least four levels
+    const int passes = path ? 2 * ((steps + 3) / 4) : (steps + kTreeLevels - 1) / kTreeLevels;
+#define SKT_OT(K_)                                                                               \
+  do {                                                                                           \
+    hipLaunchKernelGGL(k_oc_candidate_tree<K_>, dim3(grid_for(nd)), dim3(kBlock), 0, stream, nd, \
+                       f->design_ids, rho_e, dC, f->state, 1e-12, eta, rate_min, rate_max,       \
+                       move_limit, rho_min, rho_max, f->cand_tree);                              \
+    hipLaunchKernelGGL(k_oc_volume_tree<K_>, dim3(nb), dim3(kBlock), 0, stream, nd, f->row_ptr,  \
+                       f->gcol, f->w, f->cand_tree, vol, beta, beta_eta, tbe, denom, f->state,   \
+                       f->part_tree);                                                            \
+    hipLaunchKernelGGL(k_oc_bracket_tree<K_>, dim3(1), dim3(kBlock), 0, stream, (int)nb,         \
+                       f->part_tree, vol_sum, vol_frac, vol_tol, tolerance, max_iter, steps,     \
+                       eta, f->state);                                                           \
+  } while (0)
+    for (int s = 0; s < passes; ++s) {
+      if (path)
+        SKT_OT(kTreeStride);
+      else
+        SKT_OT(kTreeK);
     }
+#undef SKT_OT
     hipLaunchKernelGGL(k_oc_candidate_at, dim3(grid_for(nd)), dim3(kBlock), 0, stream, nd, rho_e,
                        dC, f->state, 1e-12, eta, rate_min, rate_max, move_limit, rho_min,
                        rho_max, rho_out);
