@@ -1186,6 +1186,55 @@ __global__ void k_restrict_xy(int fnx, int fny, int fnz, int fx, int fy, int gro
   }
 }
 
+// Pass 1 for factors of at most 3 where its rows are few: a thread per coarse
+// column and component, its up to 5 x 5 fine nodes and their flags loaded
+// unpredicated (clamped addresses) before any is used.  The kernel above waits
+// for memory at each of its taps.  The same sums in the same order.  33x17x13
+// elements, factor 3, 2 float64 columns: 15.0 to 8.2 us; 25x13x13, one float32
+// column: 7.4 to 4.9 us.
+template <typename T, int NC, int KC, bool HASW>
+__global__ void __launch_bounds__(256)
+k_restrict_xy_gather(int fnx, int fny, int fnz, int fx, int fy, int groups,
+                     const T* __restrict__ b, const T* __restrict__ w,
+                     const uint8_t* __restrict__ fixed, T* __restrict__ tbuf) {
+  const int fnnx = fnx + 1, fnny = fny + 1, fnnz = fnz + 1;
+  const int cnnx = (fnx + fx - 1) / fx + 1, cnny = (fny + fy - 1) / fy + 1;
+  const int64_t tn = (int64_t)cnnx * cnny * fnnz, fnn = (int64_t)fnnx * fnny * fnnz;
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;  // launched below 2^31
+  if (t >= tn * NC * groups) return;
+  const int d = t % NC, gn = t / NC, g = gn / (int)tn, node = gn - g * (int)tn;
+  const int row = node / cnnx, I = node - row * cnnx, k = row / cnny, J = row - k * cnny;
+  const Taps tx = coarse_taps(I, fx, fnx), ty = coarse_taps(J, fy, fny);
+  const T* bg = b + g * fnn * NC * KC;
+  const T* wg = HASW ? w + g * fnn * NC * KC : nullptr;
+  T acc[KC];
+#pragma unroll
+  for (int c = 0; c < KC; ++c) acc[c] = T(0);
+  T bv[25][KC], wv[HASW ? 25 : 1][KC];
+  uint8_t fx_[25];
+#pragma unroll
+  for (int o = 0; o < 25; ++o) {
+    const int i = min(max(tx.x + o % 5 - 2, 0), fnx), j = min(max(ty.x + o / 5 - 2, 0), fny);
+    const int64_t dof = (i + fnnx * (j + (int64_t)fnny * k)) * NC + d;
+    load_node<T, KC, KC>(bg + dof * KC, bv[o]);
+    if constexpr (HASW) load_node<T, KC, KC>(wg + dof * KC, wv[o]);
+    fx_[o] = fixed ? fixed[dof] : 0;
+  }
+#pragma unroll
+  for (int o = 0; o < 25; ++o) {
+    const int dx = o % 5 - 2, dy = o / 5 - 2;
+    const bool in = dx > -tx.wl && dx < tx.wr && dy > -ty.wl && dy < ty.wr && !fx_[o];
+    const T wy = T(1) - (dy < 0 ? (T)-dy / (T)ty.wl : (T)dy / (T)ty.wr);
+    const T wgt = (T(1) - (dx < 0 ? (T)-dx / (T)tx.wl : (T)dx / (T)tx.wr)) * wy;
+#pragma unroll
+    for (int c = 0; c < KC; ++c) {
+      const T n = acc[c] + wgt * (HASW ? bv[o][c] - wv[HASW ? o : 0][c] : bv[o][c]);
+      acc[c] = in ? n : acc[c];
+    }
+  }
+  store_node<T, KC, KC>(tbuf + ((g * tn + node) * NC + d) * KC, acc);
+}
+
 // Pass 2 (z): b_c(I, J, K) = sum_dz w(dz) t(I, J, f K + dz).  Thread: (I, J);
 // row: (K, group).
 template <typename T, int NC, int KC>
@@ -2376,18 +2425,6 @@ int mg_setup(MGData* mg, const skt_operator* op, const double* E64, const void* 
   return setup_t<float>(mg, op, E64, E, dinv0, s);
 }
 
-template <typename T, int NC, int KC>
-static void launch_restrict(const MGLevel& f, const MGLevel& c, int groups, const T* b,
-                            const T* w, const uint8_t* fixed, T* bc, hipStream_t s) {
-  T* tbuf = (T*)c.rt;
-  const RowGrid gxy = row_grid(c.nx + 1, (c.ny + 1) * (f.nz + 1) * groups);
-  hipLaunchKernelGGL((k_restrict_xy<T, NC, KC>), gxy.grid, gxy.block, 0, s, (int)f.nx, (int)f.ny,
-                     (int)f.nz, c.f[0], c.f[1], groups, b, w, fixed, tbuf);
-  const RowGrid gz = row_grid((c.nx + 1) * (c.ny + 1), (c.nz + 1) * groups);
-  hipLaunchKernelGGL((k_restrict_z<T, NC, KC>), gz.grid, gz.block, 0, s, (int)(c.nx + 1),
-                     (int)(c.ny + 1), (int)f.nz, c.f[2], groups, (const T*)tbuf, bc);
-}
-
 // SKT_MG_TRANSFERS=rowgrid forces the row-grid restriction on every level
 // (the factor-2 kernel gives the same sums; a test checks that the solves
 // agree bit for bit).
@@ -2396,15 +2433,40 @@ static bool fused_transfers_enabled() {
   return !(v && std::strcmp(v, "rowgrid") == 0);
 }
 
-// Fused restriction into level c when every factor is 2 (k_restrict222; b
-// zero at Dirichlet DOFs); with x0, also the first smoothing iterate of c
-// (coefficients cf).  Returns false, launching nothing, otherwise.
 // Largest coarse level (nodes times column groups) that k_restrict_gather
 // takes: 100x50x50 compliance and gradient 9.36 ms without it, 9.24 up to
 // 32768, 9.04 up to 131072 (its fine level too); 120x60x60 with 8 loads, whose
 // fine level has 230,000, 13.9 ms, and 14.1 with it.
 constexpr int64_t kGatherNodes = 131072;
 
+template <typename T, int NC, int KC>
+static void launch_restrict(const MGLevel& f, const MGLevel& c, int groups, const T* b,
+                            const T* w, const uint8_t* fixed, T* bc, hipStream_t s) {
+  T* tbuf = (T*)c.rt;
+  const int64_t rows = (c.nx + 1) * (c.ny + 1) * (f.nz + 1) * groups;
+  // 25 loads a thread pay while they wait for latency, not for bandwidth: the
+  // limit of the gather for factor 2, whose threads load as much
+  if (c.f[0] <= 3 && c.f[1] <= 3 && rows <= kGatherNodes && fused_transfers_enabled()) {
+    const unsigned gg = (unsigned)((rows * NC + 255) / 256);
+    if (w)
+      hipLaunchKernelGGL((k_restrict_xy_gather<T, NC, KC, true>), dim3(gg), dim3(256), 0, s,
+                         (int)f.nx, (int)f.ny, (int)f.nz, c.f[0], c.f[1], groups, b, w, fixed, tbuf);
+    else
+      hipLaunchKernelGGL((k_restrict_xy_gather<T, NC, KC, false>), dim3(gg), dim3(256), 0, s,
+                         (int)f.nx, (int)f.ny, (int)f.nz, c.f[0], c.f[1], groups, b, w, fixed, tbuf);
+  } else {
+    const RowGrid gxy = row_grid(c.nx + 1, (c.ny + 1) * (f.nz + 1) * groups);
+    hipLaunchKernelGGL((k_restrict_xy<T, NC, KC>), gxy.grid, gxy.block, 0, s, (int)f.nx, (int)f.ny,
+                       (int)f.nz, c.f[0], c.f[1], groups, b, w, fixed, tbuf);
+  }
+  const RowGrid gz = row_grid((c.nx + 1) * (c.ny + 1), (c.nz + 1) * groups);
+  hipLaunchKernelGGL((k_restrict_z<T, NC, KC>), gz.grid, gz.block, 0, s, (int)(c.nx + 1),
+                     (int)(c.ny + 1), (int)f.nz, c.f[2], groups, (const T*)tbuf, bc);
+}
+
+// Fused restriction into level c when every factor is 2 (k_restrict222; b
+// zero at Dirichlet DOFs); with x0, also the first smoothing iterate of c
+// (coefficients cf).  Returns false, launching nothing, otherwise.
 template <typename T, int NC, int KC>
 static bool launch_restrict_fused(const MGLevel& f, const MGLevel& c, int groups, const T* b,
                                   const T* w, T* bc, const double* cf, T* x0, hipStream_t s) {
