@@ -26,6 +26,52 @@ static int axis_factor(int64_t n) {
   return 1;
 }
 
+// Whether the stiffness has a null space on the free DOFs: a scalar operator
+// without mass and without Dirichlet nodes, or supports that leave a rigid
+// motion free (the rigid motions' Gram matrix over the fixed DOFs has no full
+// rank; nodes of a tet grid at their places on the grid).
+static int singular_operator(const skt_operator* op, int* singular) {
+  *singular = op->n_fixed == 0 && op->mass_a == 0.0;
+  if (op->ncomp != 3 || op->n_fixed == 0) return SKT_OK;
+  std::vector<int32_t> dofs((size_t)op->n_fixed);
+  SKT_HIP(hipMemcpy(dofs.data(), op->fixed_list, sizeof(int32_t) * dofs.size(),
+                    hipMemcpyDeviceToHost));
+  const int64_t nnx = op->nx + 1, nny = op->ny + 1;
+  const double len[3] = {op->nx * op->h[0], op->ny * op->h[1], op->nz * op->h[2]};
+  const double unit = std::max(len[0], std::max(len[1], len[2]));
+  double G[6][6] = {};
+  for (int32_t dof : dofs) {
+    const int64_t n = dof / 3;
+    const double x[3] = {(n % nnx * op->h[0] - 0.5 * len[0]) / unit,
+                         (n / nnx % nny * op->h[1] - 0.5 * len[1]) / unit,
+                         (n / (nnx * nny) * op->h[2] - 0.5 * len[2]) / unit};
+    const int d = dof % 3, e = (d + 1) % 3, f = (d + 2) % 3;
+    double m[6] = {};          // component d of the translations and of the
+    m[d] = 1.0;                // rotations about each axis (axis x position)
+    m[3 + e] = x[f];
+    m[3 + f] = -x[e];
+    for (int i = 0; i < 6; ++i)
+      for (int j = 0; j < 6; ++j) G[i][j] += m[i] * m[j];
+  }
+  // elimination with diagonal pivoting
+  bool done[6] = {};
+  const double tiny = 1e-10 * op->n_fixed;
+  for (int step = 0; step < 6; ++step) {
+    int p = -1;
+    for (int i = 0; i < 6; ++i)
+      if (!done[i] && (p < 0 || G[i][i] > G[p][p])) p = i;
+    if (G[p][p] <= tiny) {
+      *singular = 1;
+      return SKT_OK;
+    }
+    done[p] = true;
+    for (int i = 0; i < 6; ++i)
+      for (int j = 0; j < 6; ++j)
+        if (!done[i] && !done[j]) G[i][j] -= G[i][p] * G[p][j] / G[p][p];
+  }
+  return SKT_OK;
+}
+
 // Coarsening factors of a level by factors 2, 3 or 5 that divide its axes; an
 // axis is not collapsed to a single element while a longer axis (more than 5
 // elements) still coarsens: e.g. 15x5x5 -> 5x5x5, not 5x1x1.
@@ -558,10 +604,10 @@ __global__ void k_stencil_dinv(int64_t nx, int64_t ny, int64_t nz, int layout,
 }
 
 // Dense coarsest matrix (fp64, row-major, n rows padded to np with the
-// identity).
+// identity), its diagonal times `scale` (above 1 for a singular operator).
 template <int NC>
 __global__ void k_dense_asm(int64_t nx, int64_t ny, int64_t nz, const double* __restrict__ Kel,
-                            int64_t np, double* __restrict__ A) {
+                            int64_t np, double scale, double* __restrict__ A) {
   const int64_t nnx = nx + 1, nny = ny + 1;
   const int64_t n = nnx * nny * (nz + 1) * NC;
   for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < np * np;
@@ -580,7 +626,7 @@ __global__ void k_dense_asm(int64_t nx, int64_t ny, int64_t nz, const double* __
     if (ox >= -1 && ox <= 1 && oy >= -1 && oy <= 1 && oz >= -1 && oz <= 1)
       v = couple<NC>(Kel, nx, ny, nz, i, j, k, (int)ox, (int)oy, (int)oz, d, e);
     // a DOF that no free fine DOF depends on gets the identity
-    A[t] = r == c && !(v > 0.0) ? 1.0 : v;
+    A[t] = r != c ? v : v > 0.0 ? scale * v : 1.0;
   }
 }
 
@@ -1973,6 +2019,9 @@ int mg_alloc(MGData* mg, const skt_operator* op, const MGConfig& cfg, int dtype,
     set_error("grid cannot be coarsened for multigrid");
     return SKT_EINVAL;
   }
+  int singular = 0;
+  if (int stt = singular_operator(op, &singular)) return stt;
+  mg->shift = singular ? kNullShift : 0.0;
   const int NC = op->ncomp, ND = 8 * NC;
   const size_t ts = tsize(dtype);
   const int L = (int)lv.size() - 1;
@@ -2343,10 +2392,10 @@ static int setup_t(MGData* mg, const skt_operator* op, const double* E64, const 
     const int64_t np = gj_pad(n);
     if (NC == 3)
       hipLaunchKernelGGL((k_dense_asm<3>), dim3(grid_for(np * np)), dim3(kBlock), 0, g, c.nx,
-                         c.ny, c.nz, c.Kel, np, mg->Ad);
+                         c.ny, c.nz, c.Kel, np, 1.0 + mg->shift, mg->Ad);
     else
       hipLaunchKernelGGL((k_dense_asm<1>), dim3(grid_for(np * np)), dim3(kBlock), 0, g, c.nx,
-                         c.ny, c.nz, c.Kel, np, mg->Ad);
+                         c.ny, c.nz, c.Kel, np, 1.0 + mg->shift, mg->Ad);
     if (!lagged) {
       queue_gj(mg, g);
       queue_cast<T>(mg, g);

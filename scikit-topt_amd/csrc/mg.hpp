@@ -55,6 +55,14 @@ constexpr int64_t kDivideNodes = 1024;
 constexpr int kLowSteps = 2;
 constexpr double kLowRatio = 30.0;
 
+// The coarsest matrix of a singular operator (a body without enough supports,
+// conduction without Dirichlet nodes) gets this share of its diagonal on top.
+// Its last pivots are otherwise what rounding leaves of zero, 1e-12 to 1e-9 of
+// the diagonal and of either sign: 32x16x16 elements without supports broke
+// down in float64 and did not converge in 3000 mixed iterations.  The motions
+// that the shift makes too soft are a few outliers of the spectrum.
+constexpr double kNullShift = 1e-5;
+
 struct MGData {
   int dtype = -1;                     // SKT_F64 / SKT_F32 the buffers hold
   int max_cols = 0;
@@ -78,6 +86,7 @@ struct MGData {
   int degree = 2;
   double ratio = 14.0;
   int low_steps = 0;
+  double shift = 0.0;                 // kNullShift for a singular operator
   int power_iters = 20;               // steps from the hashed start vector
   int power_iters_warm = 5;           // steps from the previous set-up's vector
   uint64_t gen = 0;                   // bumped whenever the buffers are (re)allocated
