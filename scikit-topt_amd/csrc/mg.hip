@@ -26,12 +26,13 @@ static int axis_factor(int64_t n) {
   return 1;
 }
 
-// Whether the stiffness has a null space on the free DOFs: a scalar operator
-// without mass and without Dirichlet nodes, or supports that leave a rigid
+// Whether the hierarchy's operator has a null space on the free DOFs: a scalar
+// one without Dirichlet nodes and without mass (which the products of tets
+// leave out), or supports that leave a rigid
 // motion free (the rigid motions' Gram matrix over the fixed DOFs has no full
 // rank; nodes of a tet grid at their places on the grid).
 static int singular_operator(const skt_operator* op, int* singular) {
-  *singular = op->n_fixed == 0 && op->mass_a == 0.0;
+  *singular = op->n_fixed == 0 && (op->mass_a == 0.0 || op->mesh == SKT_MESH_TET4);
   if (op->ncomp != 3 || op->n_fixed == 0) return SKT_OK;
   std::vector<int32_t> dofs((size_t)op->n_fixed);
   SKT_HIP(hipMemcpy(dofs.data(), op->fixed_list, sizeof(int32_t) * dofs.size(),
