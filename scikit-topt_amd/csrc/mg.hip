@@ -34,9 +34,17 @@ static int axis_factor(int64_t n) {
 static int singular_operator(const skt_operator* op, int* singular) {
   *singular = op->n_fixed == 0 && (op->mass_a == 0.0 || op->mesh == SKT_MESH_TET4);
   if (op->ncomp != 3 || op->n_fixed == 0) return SKT_OK;
-  std::vector<int32_t> dofs((size_t)op->n_fixed);
-  SKT_HIP(hipMemcpy(dofs.data(), op->fixed_list, sizeof(int32_t) * dofs.size(),
-                    hipMemcpyDeviceToHost));
+  std::vector<int32_t> dofs;
+  if (op->fixed_list) {
+    dofs.resize((size_t)op->n_fixed);
+    SKT_HIP(hipMemcpy(dofs.data(), op->fixed_list, sizeof(int32_t) * dofs.size(),
+                      hipMemcpyDeviceToHost));
+  } else {  // tet4 operators keep the flags alone
+    std::vector<uint8_t> flag((size_t)op->n_nodes * 3);
+    SKT_HIP(hipMemcpy(flag.data(), op->fixed, flag.size(), hipMemcpyDeviceToHost));
+    for (size_t i = 0; i < flag.size(); ++i)
+      if (flag[i]) dofs.push_back((int32_t)i);
+  }
   const int64_t nnx = op->nx + 1, nny = op->ny + 1;
   const double len[3] = {op->nx * op->h[0], op->ny * op->h[1], op->nz * op->h[2]};
   const double unit = std::max(len[0], std::max(len[1], len[2]));

@@ -51,3 +51,26 @@ def test_multigrid_converges_without_supports(gpu, kind, grid, precision):
     np.testing.assert_allclose(c, _solve(t, kind, precision, "jacobi")[0], rtol=1e-6)
     if grid == (32, 16, 16):
         assert _solve(t, kind, precision, "mg")[1]["converged"]
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("kind", ["free", "rollers"])
+def test_tet_grid_without_supports(gpu, kind, precision):
+    """The same on jittered tets, whose rigid rotations the grid's
+    interpolation holds only approximately."""
+    from sktopt_amd import fea
+    from sktopt_amd.mesh import toy_problem
+    t = toy_problem.cantilever(13, 7, 9, kind="tet4", jitter=0.2, seed=2)
+    h = _task(kind, (13, 7, 9))
+    t.neumann_linear, t.dirichlet_dofs, t.dirichlet_nodes = h.forces, h.dirichlet_dofs, \
+        h.dirichlet_nodes
+    rho = np.random.default_rng(7).uniform(0.05, 1.0, t.mesh.nelements)
+    c = {}
+    for pc in ("auto", "jacobi"):
+        cfg = fea.LinearSolverConfig(rtol=1e-8, precision=precision, preconditioner=pc,
+                                     mg_max_coarse=100, maxiter=1000)
+        fem = fea.FEM_SimpLinearElasticity(t, 1e-6, solver_config=cfg)
+        U = np.zeros((fem.ndof, 1))
+        c[pc] = fem.objectives_multi_load(rho, 3.0, U)
+        assert fem.last_solve["preconditioner"] == ("mg" if pc == "auto" else "jacobi")
+    np.testing.assert_allclose(c["auto"], c["jacobi"], rtol=1e-6)
