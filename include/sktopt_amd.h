@@ -358,7 +358,9 @@ int skt_solver_destroy(skt_solver* s);
  * clamp), as skfem.enforce builds it.  U: (ndof, ncols) float64, the initial
  * guess on entry (warm start; U[D] is overwritten with F[D]) and the
  * solution on exit.
- * iters[0] = PCG iterations, iters[1] = reliable updates (0 in SKT_F64);
+ * iters[0] = PCG iterations, iters[1] = reliable updates (0 in SKT_F64), those
+ * of a multigrid solve that broke down and of Jacobi's after it together
+ * (SKT_PC_AUTO; maxiter bounds each of the two);
  * relres[c] = final ||F - K U|| / ||F|| per column (host arrays, valid on
  * return).  The copy of the solution into U is stream-ordered on `stream`
  * and may still be running when the call returns. */
@@ -375,7 +377,10 @@ int skt_solver_solve(skt_solver* s, int mode, int ncols, const double* E64,
  *                  the Dirichlet DOFs removed, Chebyshev-Jacobi smoothing of
  *                  smooth_degree steps, dense inverse on the coarsest level
  *                  (at most max_coarse DOFs);
- *   SKT_PC_AUTO    multigrid where the grid allows it, else Jacobi (default).
+ *   SKT_PC_AUTO    multigrid where the grid allows it, else Jacobi (default);
+ *                  Jacobi also where the V-cycle turns out not to be definite
+ *                  or CG breaks down with it, and, after two such solves in a
+ *                  row, until the solver is configured anew.
  * skt_solver_info reports the preconditioner the last solve used and its
  * number of levels (1 for Jacobi). */
 #define SKT_PC_JACOBI 0

@@ -1884,13 +1884,13 @@ __global__ void k_pow_scale(int64_t n, const double* __restrict__ inv, const T* 
 // Chebyshev (c1, c2) per step for the interval [beta/ratio, beta]; the last
 // level takes ratio_low.  The residual polynomial stays below 1 in magnitude,
 // and the cycle positive definite, up to beta (1 + 1/ratio): beta is chosen so
-// that this is 1.21 times the power iteration's estimate for every ratio.
-__global__ void k_cheb_coef(int nlev, int degree, double ratio, double ratio_low,
+// that this is `margin` times the power iteration's estimate for every ratio.
+__global__ void k_cheb_coef(int nlev, int degree, double ratio, double ratio_low, double margin,
                             const double* __restrict__ lam, double* __restrict__ coef) {
   const int l = threadIdx.x;
   if (l >= nlev) return;
   const double r = l > 0 && l == nlev - 1 ? ratio_low : ratio;
-  const double bmax = 1.21 / (1.0 + 1.0 / r) * lam[l];
+  const double bmax = margin / (1.0 + 1.0 / r) * lam[l];
   const double amin = bmax / r;
   const double theta = 0.5 * (bmax + amin), delta = 0.5 * (bmax - amin);
   const double sigma = theta / delta;
@@ -2087,6 +2087,11 @@ int mg_alloc(MGData* mg, const skt_operator* op, const MGConfig& cfg, int dtype,
   if (const char* rv = std::getenv("SKT_MG_RATIO")) {  // smoothing interval [lambda/r, lambda]
     const double r = std::atof(rv);
     if (r > 1.0 && r < 1000.0) mg->ratio = r;
+  }
+  mg->margin = kChebMargin;
+  if (const char* mv = std::getenv("SKT_MG_MARGIN")) {  // below 1 the cycle is not definite
+    const double m = std::atof(mv);
+    if (m > 0.0 && m <= 4.0) mg->margin = m;
   }
   mg->power_iters = cfg.power_iters;
   mg->lag = lag_enabled();
@@ -2465,7 +2470,7 @@ static int setup_t(MGData* mg, const skt_operator* op, const double* E64, const 
   }
   mg->warm = 1;
   hipLaunchKernelGGL(k_cheb_coef, dim3(1), dim3(64), 0, s, L, coef_steps(mg), mg->ratio,
-                     mg->low_steps ? std::max(mg->ratio, kLowRatio) : mg->ratio, mg->lam,
+                     mg->low_steps ? std::max(mg->ratio, kLowRatio) : mg->ratio, mg->margin, mg->lam,
                      mg->coef);
   SKT_LAUNCH_CHECK();
   // every side-stream branch joins the main stream before the set-up

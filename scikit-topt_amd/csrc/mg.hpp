@@ -55,6 +55,10 @@ constexpr int64_t kDivideNodes = 1024;
 constexpr int kLowSteps = 2;
 constexpr double kLowRatio = 30.0;
 
+// The smoothers' bound over the power iteration's estimate of lambda_max
+// (k_cheb_coef).
+constexpr double kChebMargin = 1.21;
+
 // The coarsest matrix of a singular operator (a body without enough supports,
 // conduction without Dirichlet nodes) gets this share of its diagonal on top.
 // Its last pivots are otherwise what rounding leaves of zero, 1e-12 to 1e-9 of
@@ -85,6 +89,7 @@ struct MGData {
   int warm = 0;                       // pvw holds vectors from an earlier set-up
   int degree = 2;
   double ratio = 14.0;
+  double margin = kChebMargin;
   int low_steps = 0;
   double shift = 0.0;                 // kNullShift for a singular operator
   int power_iters = 20;               // steps from the hashed start vector

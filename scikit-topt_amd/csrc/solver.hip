@@ -59,6 +59,7 @@ struct skt_solver {
   skt::MGConfig mgcfg;
   skt::MGData mg;
   int mg_possible = -1;      // -1 unknown, 0 no, 1 yes, 2 only where not asked for
+  int broken = 0;            // solves in a row whose multigrid broke down
   // optional per-launch timing of the operator apply (hipEvents on the
   // solve stream, read back at the convergence checks); only chunks that
   // start with every column live are timed, since the apply skips the work
@@ -129,7 +130,8 @@ static int mg_poll_interval() {
 }
 // scalar slots
 enum {
-  S_RZ = 0, S_PQ, S_ALPHA, S_BETA, S_RR, S_BB, S_CONV, S_TOL2, S_BAD,
+  S_RZ = 0, S_NEG, S_ALPHA, S_BETA, S_RR, S_BB, S_CONV, S_TOL2, S_BAD,
+  // S_NEG 1: r.z was negative before convergence, the preconditioner is not definite
   S_RREF,    // r.r at the last reliable update (0: no updates, float64 mode)
   S_REQ,     // 1: the column asks for a reliable update
   S_DELTA2,  // reliable-update threshold on r.r / r.r at the last update
@@ -140,6 +142,9 @@ enum {
 };
 static_assert(S_TCONV < 16, "scalar slots");
 constexpr int kMaxRestarts = 8;
+// After this many breakdowns in a row the automatic choice is Jacobi until the
+// solver is configured anew: every further try would cost both methods.
+constexpr int kMaxBroken = 2;
 
 // Blocked-layout geometry of one solve.
 struct Blk {
@@ -394,6 +399,7 @@ __global__ void k_init_final(int nb, int k, const double* __restrict__ part_rb,
     s[S_BB] = bb;
     s[S_RZ] = rz;
     s[S_TOL2] = rtol2 * bb;
+    s[S_NEG] = rz < 0.0 && rr > s[S_TOL2] ? 1.0 : 0.0;
     s[S_CONV] = (rr <= s[S_TOL2]) ? 1.0 : 0.0;
     s[S_ALPHA] = 0.0;
     s[S_BETA] = 0.0;
@@ -412,7 +418,6 @@ __global__ void k_alpha(int nb, int k, const double* __restrict__ part, double* 
   const double pq = col_sum(part, k, nb, 0, c);
   if (threadIdx.x == 0) {
     double* s = sc + c * kSc;
-    s[S_PQ] = pq;
     if (s[S_CONV] != 0.0) {
       s[S_ALPHA] = 0.0;
     } else if (!(pq > 0.0)) {  // breakdown (or NaN): stop this column
@@ -439,6 +444,7 @@ __global__ void k_beta(int nbz, const double* __restrict__ part_rz, int nbr,
       s[S_BETA] = rz / s[S_RZ];
       s[S_RZ] = rz;
       if (rr <= s[S_TOL2]) s[S_CONV] = 1.0;
+      else if (rz < 0.0) s[S_NEG] = 1.0;
       if (rr < s[S_DELTA2] * s[S_RREF]) s[S_REQ] = 1.0;
       if (rr != rr || rz != rz) { s[S_CONV] = 1.0; s[S_BAD] = 1.0; }
     }
@@ -500,6 +506,7 @@ __global__ void k_beta_replace(int nbz, const double* __restrict__ part_rz, int 
     }
     s[S_BETA] = rst ? 0.0 : rz / s[S_RZ];
     s[S_RZ] = rz;
+    if (rz < 0.0 && rr > s[S_TOL2]) s[S_NEG] = 1.0;
     s[S_RR] = rr;
     s[S_RREF] = rr;
     s[S_REQ] = 0.0;
@@ -526,6 +533,7 @@ __global__ void k_replace_final(int nb, int k, const double* __restrict__ part_r
     s[S_RST] = (rr > 4.0 * s[S_RR] || rr > s[S_RREF]) ? 1.0 : 0.0;
     s[S_RR] = rr;
     s[S_RZ] = rz;
+    if (rz < 0.0 && rr > s[S_TOL2]) s[S_NEG] = 1.0;
     s[S_RREF] = rr;
     s[S_REQ] = 0.0;
     if (s[S_BAD] != 0.0 && s[S_NRST] < kMaxRestarts) {
@@ -835,6 +843,7 @@ static int setup_precond(skt_solver* s, const Blk& b, const double* E64, const V
                          hipStream_t st) {
   s->used = SKT_PC_JACOBI;
   if (s->precond == SKT_PC_JACOBI) return SKT_OK;
+  if (s->precond == SKT_PC_AUTO && s->broken >= kMaxBroken) return SKT_OK;
   if (s->mg_possible < 0) {
     std::vector<MGLevel> lv;
     const bool grid = (s->op->mesh == SKT_MESH_HEX8 && s->op->modal_ok) ||
@@ -882,7 +891,8 @@ static int setup_precond(skt_solver* s, const Blk& b, const double* E64, const V
 
 template <typename T>
 static int solve_t(skt_solver* s, int mode, const Blk& b, const double* E64, const Vecs<T>& v,
-                   double rtol, int maxiter, double inner_rtol, int64_t* iters, hipStream_t st) {
+                   double rtol, int maxiter, double inner_rtol, int64_t* iters, bool* broke,
+                   hipStream_t st) {
   const bool mixed = mode == SKT_F32;
   const bool mg = s->used == SKT_PC_MG;
   const int64_t total = b.n * b.k;
@@ -924,6 +934,11 @@ static int solve_t(skt_solver* s, int mode, const Blk& b, const double* E64, con
     if ((stt = collect_timing(s, v.dtype, chunk))) return stt;
     const bool bad = any_flag(s, b.k, S_BAD);
     const bool all_stop = all_flag(s, b.k, S_CONV);
+    // a cycle that is not definite: where Jacobi may take over, at once
+    if (mg && s->precond == SKT_PC_AUTO && !all_stop && any_flag(s, b.k, S_NEG)) {
+      *broke = true;
+      break;
+    }
     if (!mixed) {
       if (bad) break;
       conv = all_stop;
@@ -973,8 +988,9 @@ static int solve_t(skt_solver* s, int mode, const Blk& b, const double* E64, con
     if (any_flag(s, b.k, S_BAD)) break;
     conv = all_flag(s, b.k, S_CONV);
   }
-  iters[0] = it;
-  iters[1] = updates;
+  iters[0] += it;
+  iters[1] += updates;
+  *broke = *broke || (!conv && any_flag(s, b.k, S_BAD));
   return conv ? SKT_OK : SKT_ENOCONV;
 }
 
@@ -1016,6 +1032,7 @@ int skt_solver_configure(skt_solver* s, int precond, int smooth_degree, int max_
   SKT_CHECK(smooth_degree >= 1 && smooth_degree <= 8, "smooth_degree must be in [1, 8]");
   SKT_CHECK(max_coarse >= 8 && max_coarse <= 6000, "max_coarse must be in [8, 6000]");
   s->precond = precond;
+  s->broken = 0;
   s->ready_mode = -1;
   if (s->mgcfg.degree != smooth_degree || s->mgcfg.max_coarse != max_coarse) {
     mg_free(&s->mg);
@@ -1127,19 +1144,16 @@ int skt_solver_solve(skt_solver* s, int mode, int ncols, const double* E64,
   const bool ready = s->fixed_moduli && s->ready_mode == mode && s->ready_gen == s->mg.gen;
   if (ready) s->used = s->ready_used;
   s->ready_mode = -1;  // until this solve's set-up has succeeded
-  // mg_possible 2: a grid that has multigrid only by the automatic choice, and
-  // that Jacobi would have solved; should the cycle break down there, Jacobi
-  // starts again from the caller's U
-  auto again = [&](int st1) -> bool {
-    bool bad = st1 == SKT_ENOCONV;
-    for (int c = 0; c < ncols; ++c) bad = bad || s->host[c * kSc + S_BAD] != 0.0;
-    if (!bad || s->used != SKT_PC_MG || s->mg_possible != 2) return false;
+  // Should the multigrid that the automatic choice took break down (not where
+  // it spent its iterations), Jacobi starts again from the caller's U.
+  bool broke = false;
+  auto again = [&]() -> bool {
+    if (!broke || s->used != SKT_PC_MG || s->precond != SKT_PC_AUTO) return false;
     hipLaunchKernelGGL(k_to_blocked, dim3(ge), dim3(kBlock), 0, st, n, ncols, b.kc,
                        (const double*)U, s->x64);
     hipLaunchKernelGGL(k_set_fixed, dim3(ge), dim3(kBlock), 0, st, n, b.kc, total, s->op->fixed,
                        (const double*)s->f64, s->x64);
     s->used = SKT_PC_JACOBI;
-    iters[0] = iters[1] = 0;
     return true;
   };
   if (mode == SKT_F64) {
@@ -1151,9 +1165,9 @@ int skt_solver_solve(skt_solver* s, int mode, int ncols, const double* E64,
                          s->op->fixed, s->dinv64);
       if ((stt = setup_precond<double>(s, b, E64, v, st))) return stt;
     }
-    stt = solve_t<double>(s, mode, b, E64, v, rtol, maxiter, inner_rtol, iters, st);
-    if ((stt == SKT_OK || stt == SKT_ENOCONV) && again(stt))
-      stt = solve_t<double>(s, mode, b, E64, v, rtol, maxiter, inner_rtol, iters, st);
+    stt = solve_t<double>(s, mode, b, E64, v, rtol, maxiter, inner_rtol, iters, &broke, st);
+    if (stt == SKT_ENOCONV && again())
+      stt = solve_t<double>(s, mode, b, E64, v, rtol, maxiter, inner_rtol, iters, &broke, st);
   } else {
     Vecs<float> v{s->d32, s->r32, s->p32, s->q32, s->z32, s->dinv32, E32, SKT_F32};
     if (!ready) {
@@ -1163,15 +1177,20 @@ int skt_solver_solve(skt_solver* s, int mode, int ncols, const double* E64,
                          s->op->fixed, s->dinv32);
       if ((stt = setup_precond<float>(s, b, E64, v, st))) return stt;
     }
-    stt = solve_t<float>(s, mode, b, E64, v, rtol, maxiter, inner_rtol, iters, st);
-    if ((stt == SKT_OK || stt == SKT_ENOCONV) && again(stt))
-      stt = solve_t<float>(s, mode, b, E64, v, rtol, maxiter, inner_rtol, iters, st);
+    stt = solve_t<float>(s, mode, b, E64, v, rtol, maxiter, inner_rtol, iters, &broke, st);
+    if (stt == SKT_ENOCONV && again())
+      stt = solve_t<float>(s, mode, b, E64, v, rtol, maxiter, inner_rtol, iters, &broke, st);
   }
   if (stt != SKT_OK && stt != SKT_ENOCONV) return stt;
   if (stt == SKT_OK) s->ready_mode = mode;
   s->ready_used = s->used;
   s->ready_gen = s->mg.gen;
-  if (stt == SKT_OK) {
+  // counts of multigrid solves decide how long a coarsest inverse serves
+  if (s->used != SKT_PC_MG) {
+    s->it_prev = s->it_last = 0;
+    if (broke && stt == SKT_OK) ++s->broken;
+  } else if (stt == SKT_OK) {
+    s->broken = 0;
     s->it_prev = s->it_last;
     s->it_last = iters[0];
   }

@@ -106,19 +106,48 @@ def test_mass_operator_takes_it_where_one_set_up_serves_all_solves(gpu, keep):
 
 
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
-def test_a_cycle_that_breaks_down_falls_back_to_jacobi(gpu, precision, monkeypatch):
-    """SKT_MG_RATIO = 900 leaves the smoother next to no margin above its
-    estimate, so the cycle may lose definiteness; a grid that is only halved
-    still gets its solution."""
-    monkeypatch.setenv("SKT_MG_RATIO", "900")
-    task = oprob.multiload(13, 11, 9, n_loads=2, seed=1)
+@pytest.mark.parametrize("grid", [(13, 11, 9), (16, 12, 8)])
+def test_a_cycle_that_breaks_down_falls_back_to_jacobi(gpu, grid, precision, monkeypatch):
+    """SKT_MG_MARGIN = 0.4 smooths with less than half of the largest
+    eigenvalue, so the cycle is not definite: the solve is Jacobi's, with the
+    multigrid iterations counted; after two of them Jacobi alone; a solver that
+    is configured anew tries multigrid again."""
+    from sktopt_amd import _lib
+    task = oprob.multiload(*grid, n_loads=2, seed=1)
     rho = np.where(np.random.default_rng(3).uniform(size=task.n_elements) < 0.5, 1.0, 1e-3)
-    fem = _fem(task, "elastic", precision, 1e-10, "auto", 100)
     Uo = np.zeros((task.ndof, 2))
     co = ofem.ElasticFEM(task, 1e-9).objectives_multi_load(rho, 3.0, Uo)
-    U = np.zeros((task.ndof, 2))
-    c = fem.objectives_multi_load(rho, 3.0, U)
-    np.testing.assert_allclose(c, co, rtol=1e-7)
+    ref = _fem(task, "elastic", precision, 1e-10, "jacobi", 100)
+    ref.objectives_multi_load(rho, 3.0, np.zeros((task.ndof, 2)))
+    alone = ref.last_solve["iters"]
+    monkeypatch.setenv("SKT_MG_MARGIN", "0.4")
+    fem = _fem(task, "elastic", precision, 1e-10, "auto", 100)
+
+    def solve():
+        U = np.zeros((task.ndof, 2))
+        np.testing.assert_allclose(fem.objectives_multi_load(rho, 3.0, U), co, rtol=1e-7)
+        return fem.last_solve
+    for extra in (True, True, False, False):
+        last = solve()
+        assert last["preconditioner"] == "jacobi"
+        assert (last["iters"] > alone) if extra else (last["iters"] == alone)
+    _lib.call("skt_solver_configure", fem._solver, _lib.PC_AUTO, 2, 100)
+    assert solve()["iters"] > alone
+    monkeypatch.delenv("SKT_MG_MARGIN")
+    fem = _fem(task, "elastic", precision, 1e-10, "auto", 100)
+    assert solve()["preconditioner"] == "mg"
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_spent_iterations_are_not_a_breakdown(gpu, precision):
+    """A multigrid solve that runs out of iterations ends there."""
+    from dataclasses import replace
+    task = oprob.multiload(13, 11, 9, n_loads=2, seed=1)
+    fem = _fem(task, "elastic", precision, 1e-10, "auto", 100)
+    fem.solver_config = replace(fem.solver_config, maxiter=4, on_noconv="warn")
+    fem.objectives_multi_load(_densities(task), 3.0, np.zeros((task.ndof, 2)))
+    last = fem.last_solve
+    assert last["preconditioner"] == "mg" and last["iters"] == 4 and not last["converged"]
 
 
 @pytest.mark.parametrize("grid", [(32, 16, 16), (96, 34, 34)])
