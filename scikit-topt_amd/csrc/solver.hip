@@ -859,7 +859,8 @@ static int setup_precond(skt_solver* s, const Blk& b, const double* E64, const V
                      : s->op->mass_a == 0.0 || s->fixed_moduli ? 2
                                                                : 0;
   }
-  const bool kc_ok = b.kc <= (s->op->ncomp == 3 ? 2 : 4);
+  // the column blocks that the cycle is built for; tets block all columns
+  const bool kc_ok = b.kc <= 2 || (b.kc == 4 && s->op->ncomp == 1);
   // The hierarchy leaves out Robin terms and, on tets, a mass term.  The
   // automatic choice takes it for them only where the axes divide: with strong
   // Robin facets it needs more iterations than Jacobi, whose diagonal has them

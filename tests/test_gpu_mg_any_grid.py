@@ -71,6 +71,29 @@ def test_tet_grid_of_odd_cells_matches_jacobi(gpu):
     assert np.abs(out["auto"] - out["jacobi"]).max() <= 1e-8 * np.abs(out["jacobi"]).max()
 
 
+@pytest.mark.parametrize("cells", [(7, 7, 7), (8, 8, 8)])
+@pytest.mark.parametrize("columns", [1, 2, 3, 4, 5])
+def test_tet_heat_of_any_number_of_columns(gpu, cells, columns):
+    """Tet operators take all columns as one block; the cycle is built for
+    blocks of 1, 2 and 4 scalar columns, the others are Jacobi's."""
+    from sktopt_amd import fea, mesh as pmesh
+    m = pmesh.jittered_tet(*cells, jitter=0.2, seed=3)
+    n = (cells[0] + 1) * (cells[1] + 1)
+    values = [100.0 * (c + 1) for c in range(columns)]
+    t = pmesh.LinearHeatConduction(m, np.arange(n), values, np.ones(m.nvertices), None, 1.0)
+    rho = np.random.default_rng(7).uniform(0.05, 1.0, m.nelements)
+    out = {}
+    for pc in ("auto", "jacobi"):
+        cfg = fea.LinearSolverConfig(rtol=1e-12, precision="fp64", preconditioner=pc,
+                                     mg_max_coarse=100)
+        fem = fea.FEM_SimpLinearHeatConduction(t, 1e-3, solver_config=cfg)
+        out[pc] = np.zeros((m.nvertices, columns))
+        fem.objectives_multi_load(rho, 3.0, out[pc])
+        mg = pc == "auto" and columns in (1, 2, 4)
+        assert fem.last_solve["preconditioner"] == ("mg" if mg else "jacobi")
+    assert np.abs(out["auto"] - out["jacobi"]).max() <= 1e-8 * np.abs(out["jacobi"]).max()
+
+
 def test_explicit_request_stays_refused(gpu):
     """Factors 2, 3 and 5 do not reach 100 DOFs from 13 x 11 x 7 elements."""
     task = oprob.cantilever(13, 11, 7)
