@@ -49,9 +49,11 @@ struct skt_solver {
   int inv_age = 0;
   // The operator and moduli stay as they are between solves
   // (skt_solver_fix_moduli): the diagonal and the preconditioner of the first
-  // solve in a mode serve the later ones, as long as their buffers live.
+  // solve in a mode serve the later ones, as long as their buffers live and the
+  // multigrid serves their column block as it did or did not the first one's.
   int fixed_moduli = 0;
   int ready_mode = -1, ready_used = 0;
+  bool ready_block = false;
   uint64_t ready_gen = 0;
   // preconditioner
   int precond = SKT_PC_AUTO;
@@ -580,6 +582,11 @@ static int kc_for(const skt_operator* op, int k) {
   return k % 4 == 0 ? 4 : (k % 2 == 0 ? 2 : 1);
 }
 
+// the column blocks that the V-cycle is built for; tets block all columns
+static bool mg_block(const skt_operator* op, int kc) {
+  return kc <= 2 || (kc == 4 && op->ncomp == 1);
+}
+
 // Vectors of one precision for the PCG loop.
 template <typename T>
 struct Vecs {
@@ -859,8 +866,7 @@ static int setup_precond(skt_solver* s, const Blk& b, const double* E64, const V
                      : s->op->mass_a == 0.0 || s->fixed_moduli ? 2
                                                                : 0;
   }
-  // the column blocks that the cycle is built for; tets block all columns
-  const bool kc_ok = b.kc <= 2 || (b.kc == 4 && s->op->ncomp == 1);
+  const bool kc_ok = mg_block(s->op, b.kc);
   // The hierarchy leaves out Robin terms and, on tets, a mass term.  The
   // automatic choice takes it for them only where the axes divide: with strong
   // Robin facets it needs more iterations than Jacobi, whose diagonal has them
@@ -1142,7 +1148,9 @@ int skt_solver_solve(skt_solver* s, int mode, int ncols, const double* E64,
                      (const double*)s->f64, s->x64);
   SKT_LAUNCH_CHECK();
   int stt;
-  const bool ready = s->fixed_moduli && s->ready_mode == mode && s->ready_gen == s->mg.gen;
+  const bool block = mg_block(s->op, b.kc);
+  const bool ready = s->fixed_moduli && s->ready_mode == mode && s->ready_gen == s->mg.gen &&
+                     s->ready_block == block;
   if (ready) s->used = s->ready_used;
   s->ready_mode = -1;  // until this solve's set-up has succeeded
   // Should the multigrid that the automatic choice took break down (not where
@@ -1185,6 +1193,7 @@ int skt_solver_solve(skt_solver* s, int mode, int ncols, const double* E64,
   if (stt != SKT_OK && stt != SKT_ENOCONV) return stt;
   if (stt == SKT_OK) s->ready_mode = mode;
   s->ready_used = s->used;
+  s->ready_block = block;
   s->ready_gen = s->mg.gen;
   // counts of multigrid solves decide how long a coarsest inverse serves
   if (s->used != SKT_PC_MG) {

@@ -9,7 +9,7 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("grid", [(20, 16, 14), (23, 19, 13)])  # multigrid, Jacobi
+@pytest.mark.parametrize("grid", [(20, 16, 14), (23, 19, 13)])
 def test_later_solves_equal_fresh_set_ups(gpu, grid):
     import torch
     from sktopt_amd import _lib
@@ -48,3 +48,33 @@ def test_later_solves_equal_fresh_set_ups(gpu, grid):
     for v in s.values():
         _lib.load().skt_solver_destroy(v)
     _lib.load().skt_operator_destroy(op)
+
+
+@pytest.mark.parametrize("order", [(1, 3, 1), (3, 1, 3)])
+def test_column_counts_on_a_grid_of_tets(gpu, order):
+    """Tets block all columns of a solve, and multigrid is built for one or two
+    of elasticity: each solve of the solver takes what its own count allows."""
+    import torch
+    from sktopt_amd import _lib, fea
+    from sktopt_amd.mesh import toy_problem
+    t = toy_problem.cantilever(8, 7, 6, kind="tet4", jitter=0.2, seed=2)
+    op = fea.FEM_SimpLinearElasticity(t, 1e-6)
+    n, dev = op.ndof, dict(dtype=torch.float64, device="cuda")
+    E = torch.ones(op.n_el, **dev)
+    free = 1.0 - torch.as_tensor(t.dof_fixed_mask(), device="cuda").double()[:, None]
+    F = free * torch.rand((n, 3), generator=torch.Generator(device="cuda").manual_seed(1), **dev)
+    s = C.c_void_p()
+    _lib.call("skt_solver_create", op._op, 3, C.byref(s))
+    _lib.call("skt_solver_configure", s, _lib.PC_AUTO, 2, 100)
+    _lib.call("skt_solver_fix_moduli", s, 1)
+    for k in order:
+        U, f = torch.zeros((n, k), **dev), F[:, :k].contiguous()
+        it, rr = (C.c_int64 * 2)(), (C.c_double * 3)()
+        _lib.call("skt_solver_solve", s, _lib.F64, k, E.data_ptr(), None, f.data_ptr(),
+                  U.data_ptr(), 1e-10, 5000, 0.0, it, rr, torch.cuda.current_stream().cuda_stream)
+        pc, lev = C.c_int(), C.c_int()
+        _lib.call("skt_solver_info", s, C.byref(pc), C.byref(lev))
+        assert pc.value == (_lib.PC_MG if k == 1 else _lib.PC_JACOBI) and max(rr[:k]) <= 1e-10
+        R = f - op.apply(U, E)
+        assert (R * free).norm() <= 1e-9 * f.norm()
+    _lib.load().skt_solver_destroy(s)
