@@ -1151,7 +1151,11 @@ int skt_solver_solve(skt_solver* s, int mode, int ncols, const double* E64,
   const bool block = mg_block(s->op, b.kc);
   const bool ready = s->fixed_moduli && s->ready_mode == mode && s->ready_gen == s->mg.gen &&
                      s->ready_block == block;
-  if (ready) s->used = s->ready_used;
+  if (ready) {
+    s->used = s->ready_used;
+    if (s->used == SKT_PC_MG)
+      if (int e = mg_set_timing(&s->mg, s->timing)) return e;
+  }
   s->ready_mode = -1;  // until this solve's set-up has succeeded
   // Should the multigrid that the automatic choice took break down (not where
   // it spent its iterations), Jacobi starts again from the caller's U.

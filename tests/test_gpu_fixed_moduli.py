@@ -78,3 +78,27 @@ def test_column_counts_on_a_grid_of_tets(gpu, order):
         R = f - op.apply(U, E)
         assert (R * free).norm() <= 1e-9 * f.norm()
     _lib.load().skt_solver_destroy(s)
+
+
+def test_timing_switched_between_solves(gpu):
+    """The V-cycle's timing follows the solver's also where a solve keeps the
+    set-up of an earlier one."""
+    import torch
+    from sktopt_amd import _lib
+    g = (20, 16, 14)
+    n, dev = 21 * 17 * 15, dict(dtype=torch.float64, device="cuda")
+    fixed, E = torch.zeros(n, dtype=torch.uint8, device="cuda"), torch.ones(20 * 16 * 14, **dev)
+    F, op, s = torch.rand((n, 1), **dev), C.c_void_p(), C.c_void_p()
+    _lib.call("skt_hex8_create_scalar", *g, 1.0, 1.0, 1.0, 1.0, 4.0, fixed.data_ptr(), C.byref(op))
+    _lib.call("skt_solver_create", op, 1, C.byref(s))
+    _lib.call("skt_solver_fix_moduli", s, 1)
+    for on in (0, 1, 0):
+        _lib.call("skt_solver_set_timing", s, on)
+        U, it, rr = torch.zeros((n, 1), **dev), (C.c_int64 * 2)(), (C.c_double * 1)()
+        _lib.call("skt_solver_solve", s, _lib.F64, 1, E.data_ptr(), None, F.data_ptr(),
+                  U.data_ptr(), 1e-10, 1000, 0.0, it, rr, torch.cuda.current_stream().cuda_stream)
+        ms, cnt = (C.c_double * 4)(), (C.c_int64 * 4)()
+        _lib.call("skt_solver_get_vcycle_timing", s, ms, cnt, 1)
+        assert rr[0] <= 1e-10 and (sum(cnt) > 0) == bool(on)
+    _lib.load().skt_solver_destroy(s)
+    _lib.load().skt_operator_destroy(op)
