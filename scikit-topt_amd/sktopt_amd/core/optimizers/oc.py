@@ -38,6 +38,18 @@ class OC_Config(common_density.DensityMethod_OC_Config):
 S_CHANGE, S_LMID, S_VOLERR, S_NEVAL, S_WIDTH, S_KKT, S_RSCALE, S_SCALE = range(8)
 
 
+def _saturating_multiplier(largest, rate_min, eta):
+    """The multiplier from which on every rate ``(|dC| / lambda)^eta`` is at
+    most ``rate_min`` for ``|dC| <= largest``, with 1% for rounding; infinity
+    where there is none."""
+    if not (rate_min > 0.0 and 1e-3 <= eta <= 1e3 and math.isfinite(largest)):
+        return math.inf
+    try:
+        return largest * (1.01 * rate_min ** (-1.0 / eta))
+    except OverflowError:       # beyond every bracket
+        return math.inf
+
+
 class OC_Optimizer(common_density.DensityMethod):
     def __init__(self, cfg: OC_Config, tsk):
         assert cfg.lambda_lower < cfg.lambda_upper
@@ -118,11 +130,8 @@ class OC_Optimizer(common_density.DensityMethod):
         # candidates and volumes are the same: one evaluation serves them (22
         # of about 40 with a bracket up to 1e7; as in the device bisection)
         _lib.call("skt_reduce", _lib.RED_MAXABS, nd, _dev.ptr(dC), None, _dev.ptr(b["vol"]), S)
-        saturating = float(b["vol"].item())
-        if cfg.scaling_rate_min > 0.0 and 1e-3 <= eta <= 1e3 and math.isfinite(saturating):
-            saturating *= 1.01 * float(cfg.scaling_rate_min) ** (-1.0 / eta)
-        else:
-            saturating = math.inf
+        saturating = _saturating_multiplier(float(b["vol"].item()), float(cfg.scaling_rate_min),
+                                            eta)
         saturated_error = None
         while True:
             saturated = lmid >= saturating

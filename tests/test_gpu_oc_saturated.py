@@ -77,3 +77,19 @@ def test_matches_oracle(gpu, name, form, monkeypatch):
         np.testing.assert_allclose(r[0], ref[0], rtol=1e-12)
         # sums of a few hundred terms in another order
         np.testing.assert_allclose(out.cpu().numpy(), ref[2], rtol=1e-12, atol=1e-14)
+
+
+def test_helmholtz_filter_with_a_small_exponent(gpu, tmp_path):
+    """rate_min^(-1 / eta) beyond float64: no multiplier saturates the rates,
+    and the design iteration runs as with any other exponent."""
+    from sktopt_amd import core
+    from sktopt_amd.mesh import toy_problem
+    from sktopt_amd.tools import SchedulerConfig as SC
+    const = lambda v: SC.constant(target_value=v)  # noqa: E731
+    cfg = core.OC_Config(dst_path=str(tmp_path), max_iters=5, p=const(3.0), beta=const(1.0),
+                         move_limit=const(0.2), vol_frac=const(0.4), filter_radius=const(1.5),
+                         filter_type="helmholtz", eta=const(1e-3), scaling_rate_min=0.1)
+    opt = core.OC_Optimizer(cfg, toy_problem.multiload(10, 6, 6, n_loads=1, seed=1))
+    opt.parameterize()
+    opt.optimize_steps(1)
+    assert np.isfinite(opt.rho_host()).all()
