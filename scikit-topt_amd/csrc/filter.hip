@@ -648,7 +648,8 @@ __global__ void k_oc_step(int first, int nb, const double* __restrict__ part, do
                           double* __restrict__ cand_full, double* __restrict__ rho_out) {
   __shared__ double sh[kBlock / kWave];
   __shared__ double sst[kOcState];
-  const bool done = st_in[5] != 0.0;
+  // (a saturated bracket may have taken the decisions of all max_evals)
+  const bool done = st_in[5] != 0.0 || st_in[6] >= (double)max_evals;
   double tot = 0.0;
   if (!first && !done) {
     double v = 0.0;
@@ -671,7 +672,7 @@ __global__ void k_oc_step(int first, int nb, const double* __restrict__ part, do
   }
   if (done) return;
   __syncthreads();
-  if (sst[5] != 0.0) return;
+  if (sst[5] != 0.0 || sst[6] >= (double)max_evals) return;
   const double lmid = sst[2];
   for (int64_t r = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; r < n_design;
        r += (int64_t)gridDim.x * blockDim.x) {
@@ -964,9 +965,9 @@ __global__ void k_oc_candidate_at(int64_t n_design, const double* __restrict__ r
 // (part: the last pass' volume, still to be decided on)
 __global__ void k_oc_result(int nb, const double* __restrict__ part, double vol_sum,
                             double vol_frac, double vol_tol, double tolerance, int max_iter,
-                            double* __restrict__ st, double* __restrict__ res) {
+                            int max_evals, double* __restrict__ st, double* __restrict__ res) {
   __shared__ double sh[kBlock / kWave];
-  if (part && st[5] == 0.0) {
+  if (part && st[5] == 0.0 && st[6] < (double)max_evals) {
     double v = 0.0;
     for (int i = threadIdx.x; i < nb; i += blockDim.x) v += part[i];
     const double tot = block_sum(v, sh);
@@ -1430,7 +1431,7 @@ int skt_oc_bisect(skt_filter* f, const double* rho_full, const double* rho_e,
                        dC, f->state, 1e-12, eta, rate_min, rate_max, move_limit, rho_min,
                        rho_max, rho_out);
     hipLaunchKernelGGL(k_oc_result, dim3(1), dim3(kBlock), 0, stream, 0, (const double*)nullptr,
-                       vol_sum, vol_frac, vol_tol, tolerance, max_iter, f->state, result);
+                       vol_sum, vol_frac, vol_tol, tolerance, max_iter, steps, f->state, result);
     SKT_LAUNCH_CHECK();
     return SKT_OK;
   }
@@ -1467,7 +1468,7 @@ int skt_oc_bisect(skt_filter* f, const double* rho_full, const double* rho_e,
   }
 #undef SKT_OV
   hipLaunchKernelGGL(k_oc_result, dim3(1), dim3(kBlock), 0, stream, nbv, (const double*)f->part,
-                     vol_sum, vol_frac, vol_tol, tolerance, max_iter, cur, result);
+                     vol_sum, vol_frac, vol_tol, tolerance, max_iter, steps, cur, result);
   SKT_LAUNCH_CHECK();
   return SKT_OK;
 }

@@ -93,3 +93,31 @@ def test_helmholtz_filter_with_a_small_exponent(gpu, tmp_path):
     opt.parameterize()
     opt.optimize_steps(1)
     assert np.isfinite(opt.rho_host()).all()
+
+
+@pytest.mark.parametrize("form", ["stencil", "tree", "csr"])
+def test_bracket_that_stalls_in_saturation(gpu, form, monkeypatch):
+    """A tolerance below the spacing of doubles at the bracket, whose midpoint
+    rounds to its lower end: the evaluations end at their bound, ceil(log2(
+    width / tolerance)) + 3, also where one serves them all."""
+    import torch
+    from sktopt_amd import _lib, mesh as pmesh
+    from sktopt_amd.filters import SpacialFilter
+    m = pmesh.structured_hex(6, 4, 4)
+    n = m.nelements
+    monkeypatch.setenv("SKT_OC_TREE", "0" if form == "csr" else "1")
+    f = SpacialFilter(m, np.ones(n), 1.5)
+    f.use_stencil = form == "stencil"
+    f.handle
+    l1, l2, tol = 1e-7, float(np.nextafter(1e7, np.inf)), 1e-12
+    rng = np.random.default_rng(3)
+    t = lambda v: torch.as_tensor(v, dtype=torch.float64, device="cuda")  # noqa: E731
+    rho, dC, vol = t(rng.uniform(0.05, 0.9, n)), t(-rng.uniform(0.0, 1.0, n)), t(np.ones(n))
+    out, res = torch.empty_like(rho), t(np.zeros(4))
+    _lib.call("skt_oc_bisect", f.handle, rho.data_ptr(), rho.data_ptr(), dC.data_ptr(),
+              vol.data_ptr(), float(n), 0.01, 0.2, 0.5, 1e-2, 1.0, 0.7, 1.3, 2.0, 0.5, l1, l2, tol,
+              1e-4, 1000, out.data_ptr(), res.data_ptr(), torch.cuda.current_stream().cuda_stream)
+    r = res.cpu().numpy()
+    assert int(r[2]) == int(np.ceil(np.log2((l2 - l1) / tol))) + 3 and r[3] > tol
+    expect = np.clip(rho.cpu().numpy() * 0.7, rho.cpu().numpy() - 0.2, rho.cpu().numpy() + 0.2)
+    np.testing.assert_allclose(out.cpu().numpy(), np.clip(expect, 1e-2, 1.0), rtol=1e-15)
