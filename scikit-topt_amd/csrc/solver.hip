@@ -876,7 +876,11 @@ static int setup_precond(skt_solver* s, const Blk& b, const double* E64, const V
                         (s->op->mesh == SKT_MESH_TET4 && s->op->mass_a != 0.0);
   if (!s->mg_possible || !kc_ok || (s->mg_possible == 2 && (left_out || s->precond == SKT_PC_MG))) {
     if (s->precond == SKT_PC_MG) {
-      set_error("multigrid needs a structured hex8 grid that coarsens below max_coarse DOFs");
+      set_error(!s->mg_possible ? "multigrid needs a structured hex8 grid or a grid of tets that "
+                                  "coarsens to max_coarse DOFs"
+                : !kc_ok        ? "multigrid on tets takes 1 or 2 columns, or 4 scalar ones"
+                                : "multigrid by request needs a grid whose axes the factors 2, 3 "
+                                  "and 5 divide down to max_coarse DOFs");
       return SKT_EINVAL;
     }
     return SKT_OK;

@@ -98,7 +98,7 @@ def test_explicit_request_stays_refused(gpu):
     """Factors 2, 3 and 5 do not reach 100 DOFs from 13 x 11 x 7 elements."""
     task = oprob.cantilever(13, 11, 7)
     fem = _fem(task, "elastic", "fp64", 1e-8, "mg", 100)
-    with pytest.raises(ValueError):
+    with pytest.raises(ValueError, match="factors 2, 3 and 5 divide"):
         fem.objectives_multi_load(_densities(task), 3.0, np.zeros((task.ndof, 1)))
 
 
