@@ -2488,13 +2488,16 @@ int mg_setup(MGData* mg, const skt_operator* op, const double* E64, const void* 
   return setup_t<float>(mg, op, E64, E, dinv0, s);
 }
 
-// SKT_MG_TRANSFERS=rowgrid forces the row-grid restriction on every level
-// (the factor-2 kernel gives the same sums; a test checks that the solves
-// agree bit for bit).
-static bool fused_transfers_enabled() {
+// SKT_MG_TRANSFERS=rowgrid forces the row-grid restriction on every level,
+// =tiled the kernels of large levels (row grid, and k_restrict222 where all
+// factors are 2).  All give the same sums; tests check that the solves agree
+// bit for bit.
+static bool transfers_are(const char* what) {
   const char* v = std::getenv("SKT_MG_TRANSFERS");
-  return !(v && std::strcmp(v, "rowgrid") == 0);
+  return v && std::strcmp(v, what) == 0;
 }
+static bool fused_transfers_enabled() { return !transfers_are("rowgrid"); }
+static bool gathers_enabled() { return !transfers_are("rowgrid") && !transfers_are("tiled"); }
 
 // Largest coarse level (nodes times column groups) that k_restrict_gather
 // takes: 100x50x50 compliance and gradient 9.36 ms without it, 9.24 up to
@@ -2509,7 +2512,7 @@ static void launch_restrict(const MGLevel& f, const MGLevel& c, int groups, cons
   const int64_t rows = (c.nx + 1) * (c.ny + 1) * (f.nz + 1) * groups;
   // 25 loads a thread pay while they wait for latency, not for bandwidth: the
   // limit of the gather for factor 2, whose threads load as much
-  if (c.f[0] <= 3 && c.f[1] <= 3 && rows <= kGatherNodes && fused_transfers_enabled()) {
+  if (c.f[0] <= 3 && c.f[1] <= 3 && rows <= kGatherNodes && gathers_enabled()) {
     const unsigned gg = (unsigned)((rows * NC + 255) / 256);
     if (w)
       hipLaunchKernelGGL((k_restrict_xy_gather<T, NC, KC, true>), dim3(gg), dim3(256), 0, s,
@@ -2545,7 +2548,7 @@ static bool launch_restrict_fused(const MGLevel& f, const MGLevel& c, int groups
   const int zch = (cnnz + zlen - 1) / zlen;
   const int64_t nblk = per * zch;
   const T* dc = x0 ? (const T*)c.dinv : nullptr;
-  if (c.nn * groups <= kGatherNodes) {
+  if (c.nn * groups <= kGatherNodes && gathers_enabled()) {
     const unsigned gg = (unsigned)((c.nn * NC * groups + 255) / 256);
     if (w)
       hipLaunchKernelGGL((k_restrict_gather<T, NC, KC, true>), dim3(gg), dim3(256), 0, s,

@@ -36,7 +36,7 @@ def test_solve_matches_direct(gpu, precision, rtol, ctol, name, mk, physics, max
     Uo = np.zeros((task.ndof, task.n_tasks))
     co = ofe.objectives_multi_load(rho, 3.0, Uo)
     out, its = {}, {}
-    for mode in ("fused", "rowgrid"):
+    for mode in ("fused", "tiled", "rowgrid"):
         monkeypatch.setenv("SKT_MG_TRANSFERS", mode)
         fem = _fem(task, physics, precision, rtol, "auto", max_coarse)
         U = np.zeros((task.ndof, task.n_tasks))
@@ -46,12 +46,46 @@ def test_solve_matches_direct(gpu, precision, rtol, ctol, name, mk, physics, max
         assert np.abs(U - Uo).max() <= 1e-6 * np.abs(Uo).max()
         out[mode], its[mode] = U, fem.last_solve["iters"]
     # the same sums in the same order
-    assert its["fused"] == its["rowgrid"]
-    np.testing.assert_array_equal(out["fused"], out["rowgrid"])
+    for mode in ("fused", "tiled"):
+        assert its[mode] == its["rowgrid"]
+        np.testing.assert_array_equal(out[mode], out["rowgrid"])
     fem = _fem(task, physics, precision, rtol, "jacobi", max_coarse)
     fem.objectives_multi_load(rho, 3.0, np.zeros((task.ndof, task.n_tasks)))
     print(f"[{name} {precision}] iterations {its['fused']}, Jacobi {fem.last_solve['iters']}")
     assert 2 * its["fused"] <= fem.last_solve["iters"]
+
+
+@pytest.mark.parametrize("grid,precision", [((65, 17, 503), "mixed"), ((65, 17, 251), "fp64"),
+                                            ((64, 17, 252), "mixed"), ((63, 31, 64), "fp64")])
+def test_tiled_restriction_of_large_levels(gpu, grid, precision, monkeypatch):
+    """Levels that take the tiled factor-2 kernel, with 8 columns, in chunks of
+    4, 2, 2 and 1 coarse planes; on the first three the last coarse plane is
+    alone in its chunk, at an odd end of the axis or not.  Two iterations, bit
+    for bit those of the row-grid kernels."""
+    from dataclasses import replace
+    nx, ny, nz = grid
+    node = np.arange((nx + 1) * (ny + 1) * (nz + 1)).reshape(nz + 1, ny + 1, nx + 1)
+    task = oprob.multiload(4, 4, 4, n_loads=8, seed=1)
+    from oracle import mesh as om
+    task.mesh = om.structured_hex(*grid)
+    task.dirichlet_nodes = node[0].ravel()
+    task.dirichlet_dofs = (3 * node[0].ravel()[:, None] + np.arange(3)).ravel()
+    f = np.zeros((8, node.size * 3))
+    f[np.arange(8), 3 * node[-1, :, -1][:8] + np.arange(8) % 3] = 1.0
+    f[:, ::7] += 1e-3 * np.random.default_rng(2).standard_normal(f[:, ::7].shape)
+    f[:, task.dirichlet_dofs] = 0.0
+    task.forces = list(f)
+    rho = np.random.default_rng(6).uniform(0.02, 1.0, nx * ny * nz)
+    out = {}
+    for mode in ("tiled", "rowgrid"):
+        monkeypatch.setenv("SKT_MG_TRANSFERS", mode)
+        fem = _fem(task, "elastic", precision, 1e-10, "auto")
+        fem.solver_config = replace(fem.solver_config, maxiter=2, on_noconv="warn")
+        out[mode] = np.zeros((node.size * 3, 8))
+        fem.objectives_multi_load(rho, 3.0, out[mode])
+        assert fem.last_solve["preconditioner"] == "mg" and fem.last_solve["iters"] == 2
+    assert np.abs(out["tiled"]).max() > 0
+    np.testing.assert_array_equal(out["tiled"], out["rowgrid"])
 
 
 def test_tet_grid_of_odd_cells_matches_jacobi(gpu):

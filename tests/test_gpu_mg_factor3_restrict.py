@@ -10,18 +10,21 @@ from test_gpu_multigrid import _fem
 pytestmark = pytest.mark.gpu
 
 GRIDS = {
-    "three-axes": (lambda: oprob.multiload(27, 9, 9, n_loads=2, seed=1), "elastic", 250),
-    "mixed-ragged": (lambda: oprob.multiload(33, 17, 13, n_loads=3, seed=2), "elastic", 2000),
-    "one-load": (lambda: oprob.multiload(15, 6, 9, n_loads=1, seed=3), "elastic", 300),
-    "four-loads": (lambda: oprob.multiload(18, 6, 8, n_loads=4, seed=4), "elastic", 300),
-    "heat": (lambda: oprob.heat_patch(18, patch=4), "heat", 30),
+    # task factory, physics, max_coarse, levels; factors of the level taken by 3
+    "three-axes": (lambda: oprob.multiload(27, 9, 9, n_loads=2, seed=1), "elastic", 480, 2),  # 3 3 3
+    "mixed-ragged": (lambda: oprob.multiload(33, 17, 13, n_loads=3, seed=2), "elastic", 2000,
+                     2),                                                               # 3 3 3
+    "one-load": (lambda: oprob.multiload(15, 6, 9, n_loads=1, seed=3), "elastic", 300, 2),  # 3 2 3
+    "four-loads": (lambda: oprob.multiload(18, 6, 8, n_loads=4, seed=4), "elastic", 300,
+                   2),                                                                 # 3 3 3
+    "heat": (lambda: oprob.heat_patch(18, patch=4), "heat", 30, 4),                    # 3 3 3
 }
 
 
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
 @pytest.mark.parametrize("name", GRIDS)
 def test_same_solve_as_row_grid(gpu, name, precision, monkeypatch):
-    mk, physics, max_coarse = GRIDS[name]
+    mk, physics, max_coarse, levels = GRIDS[name]
     task = mk()
     rho = np.random.default_rng(8).uniform(0.05, 1.0, task.n_elements)
     out = {}
@@ -31,6 +34,7 @@ def test_same_solve_as_row_grid(gpu, name, precision, monkeypatch):
         U = np.zeros((task.ndof, task.n_tasks))
         fem.objectives_multi_load(rho, 3.0, U)
         assert fem.last_solve["preconditioner"] == "mg"
+        assert fem.last_solve["levels"] == levels
         out[mode] = (U, fem.last_solve["iters"])
     assert out["fused"][1] == out["rowgrid"][1]
     np.testing.assert_array_equal(out["fused"][0], out["rowgrid"][0])

@@ -233,11 +233,12 @@ def test_mg_two_step_smoothing_pass_matches_separate_steps(gpu, precision, physi
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
 @pytest.mark.parametrize("physics", ["elastic", "heat"])
 def test_mg_factor2_restriction_matches_row_grid_kernels(gpu, precision, physics, monkeypatch):
-    """Restriction into a level coarsened by 2 on every axis runs as one
-    LDS-staged pass that also forms the coarse level's first smoothing
-    iterate; it sums in the order of the row-grid kernels
-    (SKT_MG_TRANSFERS=rowgrid: two separable passes, then the separate first
-    step), so the solves agree bit for bit."""
+    """Restriction into a level coarsened by 2 on every axis runs as one pass
+    that also forms the coarse level's first smoothing iterate: a gather per
+    coarse node on levels of this size, LDS-staged tiles on large ones
+    (SKT_MG_TRANSFERS=tiled).  Both sum in the order of the row-grid kernels
+    (=rowgrid: two separable passes, then the separate first step), so the
+    solves agree bit for bit."""
     if physics == "elastic":
         task, max_coarse = oprob.multiload(32, 16, 16, n_loads=2, seed=7), 100
     else:
@@ -245,15 +246,16 @@ def test_mg_factor2_restriction_matches_row_grid_kernels(gpu, precision, physics
     rng = np.random.default_rng(9)
     rho = rng.uniform(0.05, 1.0, task.n_elements)
     out = {}
-    for mode in ("fused", "rowgrid"):
+    for mode in ("fused", "tiled", "rowgrid"):
         monkeypatch.setenv("SKT_MG_TRANSFERS", mode)
         fem = _fem(task, physics, precision, 1e-10, "mg", max_coarse=max_coarse)
         U = np.zeros((task.ndof, task.n_tasks))
         fem.objectives_multi_load(rho, 3.0, U)
         assert fem.last_solve["levels"] >= 3
         out[mode] = (U, fem.last_solve["iters"])
-    assert out["fused"][1] == out["rowgrid"][1]
-    np.testing.assert_array_equal(out["fused"][0], out["rowgrid"][0])
+    for mode in ("fused", "tiled"):
+        assert out[mode][1] == out["rowgrid"][1]
+        np.testing.assert_array_equal(out[mode][0], out["rowgrid"][0])
 
 
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])

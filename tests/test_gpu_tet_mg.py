@@ -152,16 +152,16 @@ def test_tet_100x50x50_oc_iterations(gpu, tmp_path):
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
 def test_tet_mg_factor2_restriction_matches_row_grid_kernels(gpu, precision, monkeypatch):
     """The tet fine level's residual (zero at Dirichlet DOFs) is restricted
-    onto the grid hierarchy by the fused factor-2 kernel, which sums in the
-    order of the two row-grid passes (SKT_MG_TRANSFERS=rowgrid): the solves
-    agree bit for bit."""
+    onto the grid hierarchy by the fused factor-2 kernels (a gather, or tiles
+    with SKT_MG_TRANSFERS=tiled), which sum in the order of the two row-grid
+    passes (=rowgrid): the solves agree bit for bit."""
     import torch
     from sktopt_amd import fea
     to = oprob.cantilever(16, 8, 8, kind="tet4", jitter=0.2, seed=7)
     c = to.centers
     rho = np.clip(0.5 + 0.6 * np.sin(c[0] / 3.0) * np.cos(c[2] / 2.0), 1e-3, 1.0)
     out = {}
-    for mode in ("fused", "rowgrid"):
+    for mode in ("fused", "tiled", "rowgrid"):
         monkeypatch.setenv("SKT_MG_TRANSFERS", mode)
         cfg = fea.LinearSolverConfig(rtol=1e-10, precision=precision, maxiter=200000,
                                      preconditioner="mg", mg_max_coarse=100)
@@ -170,5 +170,6 @@ def test_tet_mg_factor2_restriction_matches_row_grid_kernels(gpu, precision, mon
         fem.objectives_multi_load(torch.tensor(rho, device="cuda"), 3.0, U)
         assert fem.last_solve["levels"] >= 3
         out[mode] = (U.cpu().numpy(), fem.last_solve["iters"])
-    assert out["fused"][1] == out["rowgrid"][1]
-    np.testing.assert_array_equal(out["fused"][0], out["rowgrid"][0])
+    for mode in ("fused", "tiled"):
+        assert out[mode][1] == out["rowgrid"][1]
+        np.testing.assert_array_equal(out[mode][0], out["rowgrid"][0])
