@@ -2502,17 +2502,39 @@ static bool gathers_enabled() { return !transfers_are("rowgrid") && !transfers_a
 // Largest coarse level (nodes times column groups) that k_restrict_gather
 // takes: 100x50x50 compliance and gradient 9.36 ms without it, 9.24 up to
 // 32768, 9.04 up to 131072 (its fine level too); 120x60x60 with 8 loads, whose
-// fine level has 230,000, 13.9 ms, and 14.1 with it.
+// fine level has 230,000, 13.9 ms, and 14.1 with it.  Kernel times at the limit,
+// gather against tiles: 3 components, 2 columns, 125,000 nodes: 12.8 and 14.2 us
+// in float32, 20.4 and 26.5 in float64; scalar, 69,000 nodes: 1 float32 column
+// 5.0 and 6.0 us (36,000 nodes), 4 columns 6.8 and 8.3.
 constexpr int64_t kGatherNodes = 131072;
+
+// Four float64 columns are 32 bytes a load: with w a thread's 27 nodes no longer
+// fit in registers (17,000 scalar nodes: 12.6 us, tiles 9.2; 800 nodes: 10.4 and
+// 7.6), and without it they do better on small levels only (36,000 nodes: 8.0
+// and 10.7 us; 69,000: 12.2 and 11.8).
+template <typename T, int KC>
+static bool gather_fits(int64_t nodes, bool has_w) {
+  constexpr int bytes = (int)sizeof(T) * KC;
+  return bytes <= 16 ? nodes <= kGatherNodes : !has_w && nodes <= kGatherNodes / 2;
+}
 
 template <typename T, int NC, int KC>
 static void launch_restrict(const MGLevel& f, const MGLevel& c, int groups, const T* b,
                             const T* w, const uint8_t* fixed, T* bc, hipStream_t s) {
   T* tbuf = (T*)c.rt;
   const int64_t rows = (c.nx + 1) * (c.ny + 1) * (f.nz + 1) * groups;
-  // 25 loads a thread pay while they wait for latency, not for bandwidth: the
-  // limit of the gather for factor 2, whose threads load as much
-  if (c.f[0] <= 3 && c.f[1] <= 3 && rows <= kGatherNodes && gathers_enabled()) {
+  // 25 loads a thread pay while they wait for latency, not for bandwidth (the
+  // limit of the gather for factor 2, whose threads load as much), and where
+  // most of them are used: 28x28x82 scalar rows by factor 3, 7.0 us against
+  // 12.8, 12x7x14 with 6 float64 values 8.8 and 14.9.  With factors of 2 and 1,
+  // on plates, the fine level with its Dirichlet flags is faster by rows (400 x
+  // 320 elements: 10.3 us against 8.0; 300 x 280 coarsened in x only: 10.8 and
+  // 4.8), a level coarsened by 2 in x and y without flags slightly slower
+  // (50 x 40 coarse elements: 4.7 and 5.4).
+  const bool three = c.f[0] == 3 || c.f[1] == 3;
+  const bool used = c.f[0] <= 3 && c.f[1] <= 3 &&
+                    (three || (c.f[0] == 2 && c.f[1] == 2 && !fixed));
+  if (used && gather_fits<T, KC>(rows, w != nullptr) && gathers_enabled()) {
     const unsigned gg = (unsigned)((rows * NC + 255) / 256);
     if (w)
       hipLaunchKernelGGL((k_restrict_xy_gather<T, NC, KC, true>), dim3(gg), dim3(256), 0, s,
@@ -2548,7 +2570,7 @@ static bool launch_restrict_fused(const MGLevel& f, const MGLevel& c, int groups
   const int zch = (cnnz + zlen - 1) / zlen;
   const int64_t nblk = per * zch;
   const T* dc = x0 ? (const T*)c.dinv : nullptr;
-  if (c.nn * groups <= kGatherNodes && gathers_enabled()) {
+  if (gather_fits<T, KC>(c.nn * groups, w != nullptr) && gathers_enabled()) {
     const unsigned gg = (unsigned)((c.nn * NC * groups + 255) / 256);
     if (w)
       hipLaunchKernelGGL((k_restrict_gather<T, NC, KC, true>), dim3(gg), dim3(256), 0, s,
