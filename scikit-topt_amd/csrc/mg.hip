@@ -2492,12 +2492,11 @@ int mg_setup(MGData* mg, const skt_operator* op, const double* E64, const void* 
 // =tiled the kernels of large levels (row grid, and k_restrict222 where all
 // factors are 2).  All give the same sums; tests check that the solves agree
 // bit for bit.
-static bool transfers_are(const char* what) {
+enum Transfers { kGathers, kTiled, kRowGrid };
+static Transfers transfers() {
   const char* v = std::getenv("SKT_MG_TRANSFERS");
-  return v && std::strcmp(v, what) == 0;
+  return !v ? kGathers : !std::strcmp(v, "rowgrid") ? kRowGrid : !std::strcmp(v, "tiled") ? kTiled : kGathers;
 }
-static bool fused_transfers_enabled() { return !transfers_are("rowgrid"); }
-static bool gathers_enabled() { return !transfers_are("rowgrid") && !transfers_are("tiled"); }
 
 // Largest coarse level (nodes times column groups) that k_restrict_gather
 // takes: 100x50x50 compliance and gradient 9.36 ms without it, 9.24 up to
@@ -2534,7 +2533,7 @@ static void launch_restrict(const MGLevel& f, const MGLevel& c, int groups, cons
   const bool three = c.f[0] == 3 || c.f[1] == 3;
   const bool used = c.f[0] <= 3 && c.f[1] <= 3 &&
                     (three || (c.f[0] == 2 && c.f[1] == 2 && !fixed));
-  if (used && gather_fits<T, KC>(rows, w != nullptr) && gathers_enabled()) {
+  if (used && gather_fits<T, KC>(rows, w != nullptr) && transfers() == kGathers) {
     const unsigned gg = (unsigned)((rows * NC + 255) / 256);
     if (w)
       hipLaunchKernelGGL((k_restrict_xy_gather<T, NC, KC, true>), dim3(gg), dim3(256), 0, s,
@@ -2558,7 +2557,8 @@ static void launch_restrict(const MGLevel& f, const MGLevel& c, int groups, cons
 template <typename T, int NC, int KC>
 static bool launch_restrict_fused(const MGLevel& f, const MGLevel& c, int groups, const T* b,
                                   const T* w, T* bc, const double* cf, T* x0, hipStream_t s) {
-  if (c.f[0] != 2 || c.f[1] != 2 || c.f[2] != 2 || !fused_transfers_enabled()) return false;
+  const Transfers how = transfers();
+  if (c.f[0] != 2 || c.f[1] != 2 || c.f[2] != 2 || how == kRowGrid) return false;
   const int tiles_x = (int)((c.nx + 1 + kR2I - 1) / kR2I);
   const int tiles_y = (int)((c.ny + 1 + kR2J - 1) / kR2J);
   const int cnnz = (int)(c.nz + 1);
@@ -2570,7 +2570,7 @@ static bool launch_restrict_fused(const MGLevel& f, const MGLevel& c, int groups
   const int zch = (cnnz + zlen - 1) / zlen;
   const int64_t nblk = per * zch;
   const T* dc = x0 ? (const T*)c.dinv : nullptr;
-  if (gather_fits<T, KC>(c.nn * groups, w != nullptr) && gathers_enabled()) {
+  if (how == kGathers && gather_fits<T, KC>(c.nn * groups, w != nullptr)) {
     const unsigned gg = (unsigned)((c.nn * NC * groups + 255) / 256);
     if (w)
       hipLaunchKernelGGL((k_restrict_gather<T, NC, KC, true>), dim3(gg), dim3(256), 0, s,
