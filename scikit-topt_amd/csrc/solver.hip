@@ -147,6 +147,10 @@ constexpr int kMaxRestarts = 8;
 // After this many breakdowns in a row the automatic choice is Jacobi until the
 // solver is configured anew: every further try would cost both methods.
 constexpr int kMaxBroken = 2;
+// A cycle that is slightly indefinite mostly converges all the same (1.5M
+// jittered tets, first solve, estimate of lambda_max too low: 36 iterations in
+// place of 24, Jacobi 2088); one that has not by then is given up.
+constexpr int64_t kNegIters = 200;
 
 // Blocked-layout geometry of one solve.
 struct Blk {
@@ -945,8 +949,9 @@ static int solve_t(skt_solver* s, int mode, const Blk& b, const double* E64, con
     if ((stt = collect_timing(s, v.dtype, chunk))) return stt;
     const bool bad = any_flag(s, b.k, S_BAD);
     const bool all_stop = all_flag(s, b.k, S_CONV);
-    // a cycle that is not definite: where Jacobi may take over, at once
-    if (mg && s->precond == SKT_PC_AUTO && !all_stop && any_flag(s, b.k, S_NEG)) {
+    // a cycle that is not definite, where Jacobi may take over
+    if (mg && s->precond == SKT_PC_AUTO && !all_stop && it >= kNegIters &&
+        any_flag(s, b.k, S_NEG)) {
       *broke = true;
       break;
     }
