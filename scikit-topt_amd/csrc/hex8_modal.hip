@@ -649,10 +649,11 @@ static ModalGrid modal_grid(const skt_operator* op, int k, int kc_block) {
   // Small grids: a launch lasts as long as one workgroup's walk through its
   // chunk (2 to 3 us a layer), so shorter chunks down to single planes are
   // taken until there are two workgroups per CU; the layers computed twice run
-  // on CUs that would be idle.  The 40x20x20 apply with 8 float32 columns went
-  // from 19 to 8 us, an OC iteration there from 5.57 to 4.67 ms; a target of
-  // 256 workgroups gave 4.86 ms, 1024 made 66x36x28 (3 float64 columns)
-  // slower, 8.5 to 9.2 ms.
+  // on CUs that would be idle.  The 40x20x20 apply with 8 float32 columns goes
+  // from 19.6 to 11.5 us, an OC iteration there from 4.55 to 3.71 ms (a target of
+  // 256 workgroups: 3.86; 1024: 3.71), a solve on 33x17x13 with 2 float64 columns
+  // from 3.99 to 3.00 ms.  1024 costs more where 512 are there: 66x36x28, 3
+  // float64 columns, 5.58 to 6.10 ms, 75x45x30, 3 float32 ones, 7.76 to 8.17.
   while (g.lz > 1 && per * ((nnz + g.lz - 1) / g.lz) < 512) --g.lz;
   g.nzc = (int)((nnz + g.lz - 1) / g.lz);
   g.nblocks = per * g.nzc;

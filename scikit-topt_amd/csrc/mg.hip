@@ -163,8 +163,9 @@ bool mg_plan(const skt_operator* op, const MGConfig& cfg, std::vector<MGLevel>* 
     // them all does not: the largest such level.  One more halved level would
     // leave a much smaller coarsest one, and the exact solve is what catches
     // the error of stiff members in voids: 120x60x60, 8 loads, mixed, with
-    // 10x8x5 elements in place of 15x8x8 and 8x4x4 takes 24 PCG iterations
-    // per solve instead of 29 (18.6 against 21.2 ms per OC iteration).
+    // 10x8x5 elements in place of 15x8x8 and 8x4x4 takes 23 PCG iterations
+    // per solve instead of 28 (16.0 against 19.2 ms per OC iteration); 100x50x50
+    // 7.9 against 9.6 ms, 33x17x13 3.0 against 4.0, 75x45x30 the same.
     if (c.ndof > cfg.max_coarse && f.nn > kDivideNodes && !few) {
       const int64_t n3[3] = {f.nx, f.ny, f.nz};
       int64_t best = 0;
@@ -2114,10 +2115,11 @@ static int level_apply(MGData* mg, const skt_operator* op, const void* E, int l,
   // Chebyshev step: 9.7 to 8.9 us on 50x25x25 elements, 6.2 to 4.7 us on
   // 25x13x13), or where the tiles with GMT groups are fewer than the CUs
   // (20x10x10 elements, 8 float32 columns: 72 workgroups, 7.1 us; 288 with one
-  // group each, 5.2 us).  With more workgroups the coefficients' second and
-  // third read costs more: at a limit of 512, 120x60x60 with 8 loads took 15.6
-  // instead of 14.6 ms per OC iteration, 66x36x28 with 3 loads 6.75 instead of
-  // 6.53.
+  // group each, 5.2 us).  40x20x20, 8 loads: 3.98 to 3.71 ms per OC iteration,
+  // 75x45x30, 3 loads: 8.34 to 7.75 ms per solve.  With more workgroups the
+  // coefficients' second and third read costs more: at a limit of 512, 120x60x60
+  // with 8 loads takes 17.1 instead of 15.9 ms, 66x36x28 with 3 loads 5.82
+  // instead of 5.59, though 75x45x30 takes 7.57.
   constexpr int GMT = sizeof(T) == 4 ? 4 : 2;  // <= 62 KB of LDS for NC * KC = 6
   const TileShape ts = tile_shape(v.layout);
   const int64_t tiles = v.layout == ST_NODE ? 0 : st_tiles(v.nx, v.ny, v.nz, ts);
@@ -2499,9 +2501,8 @@ static Transfers transfers() {
 }
 
 // Largest coarse level (nodes times column groups) that k_restrict_gather
-// takes: 100x50x50 compliance and gradient 9.36 ms without it, 9.24 up to
-// 32768, 9.04 up to 131072 (its fine level too); 120x60x60 with 8 loads, whose
-// fine level has 230,000, 13.9 ms, and 14.1 with it.  Kernel times at the limit,
+// takes.  Limits of 32768 and 262144 change the time of a design iteration or
+// solve by less than 1% (40x20x20 to 120x60x60); kernel times near the limit,
 // gather against tiles: 3 components, 2 columns, 125,000 nodes: 12.8 and 14.2 us
 // in float32, 20.4 and 26.5 in float64; scalar, 69,000 nodes: 1 float32 column
 // 5.0 and 6.0 us (36,000 nodes), 4 columns 6.8 and 8.3.

@@ -48,10 +48,10 @@ constexpr int64_t kDivideNodes = 1024;
 
 // In elasticity the last level above the coarsest takes kLowSteps more
 // smoothing steps than the others, on the interval [lambda/kLowRatio, lambda]: its applies cost
-// little beside the fine level's (120x60x60, 8 loads, mixed: 15.5 ms per OC
-// iteration at 20 PCG iterations, against 18.6 at 24 with two steps on
-// [lambda/10, lambda] everywhere; 6 steps gave 15.0 there, but more time on
-// small grids and, now and then, a cycle that is not positive definite).
+// little beside the fine level's.  120x60x60, 8 loads, mixed: 16.0 ms per OC
+// iteration at 23 PCG iterations on average, 18.7 at 29 without them, 15.3 at 21
+// with four more; 75x45x30, 3 loads: 7.8, 8.3 and 8.0 ms; 40x20x20, 8 loads,
+// whose levels are all small: 3.7, 3.6 and 3.9.
 constexpr int kLowSteps = 2;
 constexpr double kLowRatio = 30.0;
 
@@ -130,9 +130,10 @@ enum { MG_T_CHEB0 = 0, MG_T_RESID = 1, MG_T_CHEB = 2, MG_T_CHEB_DOT = 3 };
 struct MGConfig {
   int degree = 2;          // Chebyshev steps per smoothing
   int max_coarse = 2000;   // coarsest level at most this many DOFs
-  // smoothing interval [lambda/ratio, lambda]: 14 in elasticity (10 and 20
-  // gave 16.4 and 15.7 ms per OC iteration at 120x60x60, 8 loads, 14 gave
-  // 15.5; 30 needs up to 150 iterations where the design has just changed)
+  // smoothing interval [lambda/ratio, lambda].  With the margin above it
+  // (k_cheb_coef) little depends on it: 10, 14, 20 and 30 give 15.9, 16.0, 16.1
+  // and 16.1 ms per OC iteration at 120x60x60 with 8 loads, and 7.7, 7.8, 7.9 and
+  // 8.1 ms per solve at 75x45x30 with 3
   double ratio = 14.0, ratio_scalar = 10.0;
   int power_iters = 20;
 };
